@@ -21,8 +21,13 @@
 // Scales (per column and K group) multiply the f32 partial sums; biases and
 // the SwiGLU run in the epilogue.
 //
-// k_expert_simple — VALU fallback for every other case (int4, small
-// groups): one thread per (row, column), f32 fma per group, then × scale.
+// Where the rows per expert or the weights' form ask for it, k_expert_tile
+// (expert_tile.hip) or the grouped GEMM (gemm*.hip) runs instead: the rules
+// are at expert_tile_rows and gemm_min_rows.
+//
+// k_expert_simple — VALU fallback for what is left (scale groups that are
+// not a multiple of 32, int4 with a K or an alignment k_expert_tile does not
+// take): one thread per (row, column), f32 fma per group, then × scale.
 #include <stdlib.h>
 
 #include "moe_internal.h"
@@ -895,15 +900,33 @@ int launch_mode(const ExpertArgs &ea, const ExpertKArgs &p, hipStream_t s) {
 
 }  // namespace
 
+// Where the grouped GEMM's 128-row tiles and once-converted weights beat
+// k_expert_tile's 64-row ones (µs, GEMM against tile, rows per expert):
+//   layers with f16 x: 2048 × 1408 64 rows 229, 224; 80 rows 243, 277; 640
+//     rows 1065, 1369. Short K or N never: its ring and 256-column tiles
+//     do not pay off (640 × 640 96 rows 154, 139; 640 rows 590, 569).
+//   layers with f32 x: from 64 rows, as callers have had it. The tile kernel
+//     is faster there too (640 × 640 64 rows 156, 126), but its f32 act and
+//     this path's f16-pair act differ by 5e-6 of the result, more than the
+//     2e-6 that results may move by.
+//   moe_up alone, f16 x: 640 × 640 96 rows 70, 78; 256 rows 123, 131.
+//   moe_up (f32 x) and moe_down alone: 2048 × 1408 128 rows 367, 269 and 193,
+//     161; 512 rows 893, 881 and 483, 491; 640 × 640 always the tile kernel.
+int gemm_min_rows(bool x_f16, int K, int N, bool layer) {
+  const bool wide = K >= 1024 && N >= 1024;
+  if (x_f16) return wide || !layer ? 80 : INT32_MAX;
+  return layer ? 64 : wide ? 512 : INT32_MAX;
+}
+
 bool expert_uses_gemm(const ExpertArgs &ea) {
-  // Prefill shapes (≥ 64 rows per expert on average): the grouped GEMM.
   const int max_active = ea.E < ea.A ? ea.E : ea.A;
-  const bool want_gemm = ea.A >= 64 * max_active;
-  return ea.calls == 1 && want_gemm && gemm_eligible(ea);
+  // Arguments k_expert_tile does not take: from 64 rows an expert.
+  const int64_t rows = expert_tile_eligible(ea) ? ea.gemm_rows : 64;
+  return ea.calls == 1 && ea.A >= rows * max_active && gemm_eligible(ea);
 }
 
 bool expert_stages_norm(const ExpertArgs &ea) {
-  return ea.mode == MODE_UP && !expert_uses_gemm(ea) && ea.bits == 8 &&
+  return ea.mode == MODE_UP && !ea.tile_rows && !expert_uses_gemm(ea) && ea.bits == 8 &&
          (ea.g == ea.K || ea.g % 32 == 0);
 }
 
@@ -932,6 +955,7 @@ int launch_expert(const ExpertArgs &ea, const DispatchBufs &db, hipStream_t s) {
   MOE_NONNULL(db.meta);
   if (db.E != ea.E || db.A != ea.A)
     return moe_fail(MOE_EXECUTION_FAILED, "expert: dispatch workspace sized for another shape");
+  if (ea.tile_rows) return launch_expert_tile(ea, db, s);
   if (expert_uses_gemm(ea)) return launch_expert_gemm(ea, db, s);
   ExpertKArgs p;
   p.sorted = ea.dispatch_order;

@@ -490,17 +490,11 @@ extern "C" int moe_up(moe_ctx *ctx, const void *x, moe_dtype x_dtype, const floa
   REQUIRE(x && route && act, "moeUp: NULL tensor");
   LayerWs L;
   if ((rc = plan_ws(ctx, 1, T, k, E, 0, 0, 0, 0, L))) return rc;
-  {
-    ProfScope ps(ctx, PG_DISPATCH);
-    if ((rc = launch_dispatch(route, 0, T, E, k, 1, TILE_M, L.db, ctx->stream))) return rc;
-  }
-  // Rows of ids that are not experts stay zero (the reference leaves them
-  // undefined).
-  if ((rc = launch_zero(act, (size_t)T * k * N, ctx->stream))) return rc;
   ExpertArgs ea{};
   ea.mode = MODE_UP;
   ea.a = x;
   ea.a_dtype = x_dtype;
+  ea.gemm_rows = gemm_min_rows(x_dtype == MOE_F16, K, N, false);
   ea.a_row_div = k;
   ea.route = route;
   ea.k = k;
@@ -514,6 +508,15 @@ extern "C" int moe_up(moe_ctx *ctx, const void *x, moe_dtype x_dtype, const floa
   ea.out = act;
   ea.A = T * k;
   ea.calls = 1;
+  ea.tile_rows = expert_tile_rows(ea);
+  ea.tile_m = ea.tile_rows ? ea.tile_rows : TILE_M;
+  {
+    ProfScope ps(ctx, PG_DISPATCH);
+    if ((rc = launch_dispatch(route, 0, T, E, k, 1, ea.tile_m, L.db, ctx->stream))) return rc;
+  }
+  // Rows of ids that are not experts stay zero (the reference leaves them
+  // undefined).
+  if ((rc = launch_zero(act, (size_t)T * k * N, ctx->stream))) return rc;
   {
     ProfScope ps(ctx, PG_UP);
     if ((rc = launch_expert(ea, L.db, ctx->stream))) return rc;
@@ -545,13 +548,16 @@ extern "C" int moe_down(moe_ctx *ctx, const float *act, const float *route,
   ea.g = group_size;
   ea.A = T * k;
   ea.calls = 1;
+  ea.gemm_rows = gemm_min_rows(false, K, N, false);
   ea.parts = expert_uses_gemm(ea) ? gemm_down_parts(ea) : 1;
+  ea.tile_rows = expert_tile_rows(ea);
+  ea.tile_m = ea.tile_rows ? ea.tile_rows : TILE_M;
   LayerWs L;
   if ((rc = plan_ws(ctx, 1, T, k, E, 0, 0, 0, (size_t)ea.parts * T * k * N, L))) return rc;
   ea.out = L.y;
   {
     ProfScope ps(ctx, PG_DISPATCH);
-    if ((rc = launch_dispatch(route, 0, T, E, k, 1, TILE_M, L.db, ctx->stream))) return rc;
+    if ((rc = launch_dispatch(route, 0, T, E, k, 1, ea.tile_m, L.db, ctx->stream))) return rc;
   }
   {
     ProfScope ps(ctx, PG_DOWN);
@@ -604,10 +610,11 @@ static int layer_impl(const char *op, moe_ctx *ctx, int calls, const moe_call_st
   const int A = T * k;
   // Expert products first (without buffers), so the workspace is sized for
   // the path they take.
-  ExpertArgs up{};
+  ExpertArgs up{}, dn{};
   up.mode = MODE_UP;
   up.a = x;
   up.a_dtype = x_dtype;
+  up.gemm_rows = dn.gemm_rows = gemm_min_rows(x_dtype == MOE_F16, d, I, true);
   up.a_cs = st->x;
   up.a_row_div = k;
   up.k = k;
@@ -627,7 +634,6 @@ static int layer_impl(const char *op, moe_ctx *ctx, int calls, const moe_call_st
   up.out_cs = (int64_t)A * I;
   up.A = A;
   up.calls = calls;
-  ExpertArgs dn{};
   dn.mode = MODE_DOWN;
   dn.a_dtype = MOE_F32;
   dn.a_cs = (int64_t)A * I;
@@ -644,6 +650,13 @@ static int layer_impl(const char *op, moe_ctx *ctx, int calls, const moe_call_st
   dn.g = group_size_down;
   dn.A = A;
   dn.calls = calls;
+  up.tile_rows = expert_tile_rows(up);
+  dn.tile_rows = expert_tile_rows(dn);
+  if (up.tile_rows && dn.tile_rows) dn.tile_rows = up.tile_rows;
+  // The dispatch counts M-tiles in the row tile both products use, else in
+  // the grouped GEMM's (k_expert_tile then splits them).
+  const int tile_m = up.tile_rows && up.tile_rows == dn.tile_rows ? up.tile_rows : TILE_M;
+  up.tile_m = dn.tile_m = tile_m;
   // Both products on the grouped GEMM: act stays in dispatch order, so down
   // streams each tile's rows contiguously instead of gathering them; down
   // may split K in two partial products, which the combine adds.
@@ -709,7 +722,7 @@ static int layer_impl(const char *op, moe_ctx *ctx, int calls, const moe_call_st
     up.fr_b = b_router;
     up.fr_b_cs = st->router_b;
     up.fr_J = Jr;
-    up.fr_tile_m = TILE_M;
+    up.fr_tile_m = tile_m;
   }
   up.out = L.act;
   dn.a = L.act;
@@ -721,11 +734,11 @@ static int layer_impl(const char *op, moe_ctx *ctx, int calls, const moe_call_st
                   route_cs, L.partial, T, d, E, k, calls,
                   stage_norm ? norm->weight : nullptr, norm ? norm->eps : 0.f,
                   stage_norm ? (float *)L.xn : nullptr, fuse_route ? 1 : 0};
-    if ((rc = launch_router_topk(ra, &L.db, TILE_M, &dispatched, s))) return rc;
+    if ((rc = launch_router_topk(ra, &L.db, tile_m, &dispatched, s))) return rc;
   }
   if (!dispatched) {
     ProfScope ps(ctx, PG_DISPATCH, timing);
-    if ((rc = launch_dispatch(route, route_cs, T, E, k, calls, TILE_M, L.db, s))) return rc;
+    if ((rc = launch_dispatch(route, route_cs, T, E, k, calls, tile_m, L.db, s))) return rc;
   }
   {
     ProfScope ps(ctx, PG_UP, timing);

@@ -215,6 +215,13 @@ struct ExpertArgs {
   int64_t fr_b_cs;
   int fr_J;
   int fr_tile_m;
+  // Rows per tile when these arguments run on k_expert_tile (expert_tile_rows;
+  // 0: they do not), and the M-tile rows the dispatch counted with.
+  int tile_rows;
+  int tile_m;
+  // Rows per expert (average) from which the grouped GEMM takes over from
+  // k_expert_tile (gemm_min_rows, one value for both products of a layer).
+  int gemm_rows;
 };
 
 int launch_expert(const ExpertArgs &ea, const DispatchBufs &db, hipStream_t s);
@@ -237,6 +244,14 @@ int gemm_down_parts(const ExpertArgs &ea);
 bool gemm_i8_down_eligible(const ExpertArgs &dn);
 // The direct-weight up GEMM (gemm_wide.hip) takes these arguments.
 bool gemm_wide_eligible(const ExpertArgs &ea);
+// Rows per tile (16, 32 or 64) when k_expert_tile (expert_tile.hip) takes
+// these arguments, else 0.
+int expert_tile_rows(const ExpertArgs &ea);
+bool expert_tile_eligible(const ExpertArgs &ea);
+// ExpertArgs::gemm_rows for products with K and N columns; `layer` for the
+// two products of a layer, whose act has a form of its own on the GEMM.
+int gemm_min_rows(bool x_f16, int K, int N, bool layer);
+int launch_expert_tile(const ExpertArgs &ea, const DispatchBufs &db, hipStream_t s);
 int64_t gemm_i8_act_bytes(int A, int E, int K);
 int launch_expert_gemm(const ExpertArgs &ea, const DispatchBufs &db, hipStream_t s);
 // Fills n floats with 0 (a kernel, not hipMemsetAsync, so a captured graph

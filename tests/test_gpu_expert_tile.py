@@ -1,0 +1,154 @@
+"""k_expert_tile (expert_tile.hip): row tiles of 16, 32 and 64 rows, each A
+form (f16, f32 as f16 hi + lo, f32 as three bf16 planes under int4 weights),
+plain and group scales, against the oracle's f64 products; f32's whole range
+under int4 weights; infinities and NaN stay in their rows."""
+import numpy as np
+import pytest
+import torch
+
+import runntime_amd as rt
+from oracle import ref
+
+from runntime_amd.synth import MoeConfig, make_inputs
+from tests.helpers import assert_close, random_quant_weight
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+# (T, K, N, E, g, k): rows per expert from 1 to a second 64-row tile, K one
+# 32-wide step past a piece or a ring turn, N with a partial unit group, a
+# partial column block and a wavefront without columns.
+SHAPES = [(1, 32, 8, 3, 32, 2), (5, 96, 72, 4, 32, 2), (40, 160, 136, 8, 32, 2),
+          (60, 288, 264, 6, 96, 2), (129, 640, 200, 4, 640, 2), (70, 352, 64, 2, 352, 1),
+          (260, 416, 520, 4, 416, 1), (33, 1408, 68, 1, 64, 1), (90, 64, 640, 128, 64, 4)]
+
+
+def _route(T, E, k, seed):
+    """Distinct random experts per token; slot 0 of every seventh token names none."""
+    rng = np.random.default_rng(seed)
+    ids = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.float32)
+    ids[3::7, 0] = -1.0
+    gates = rng.uniform(0.1, 1.0, (T, k)).astype(np.float32)
+    return np.concatenate([ids, gates], 1)
+
+
+def _weight(E, K, N, g, bits, seed):
+    q, sc = random_quant_weight(E, K, N, bits, g, seed)
+    bias = ref.lcg_f32(E * N, seed + 2).reshape(E, N)
+    words = rt.pack_expert_weights(q, bits)
+    dev = rt.QuantExpertWeight(
+        rt.QuantW(torch.from_numpy(words.view(np.int32)).to(DEV), (E * K, N)),
+        torch.from_numpy(sc).to(DEV), torch.from_numpy(bias).to(DEV))
+    w = q.astype(np.float64) * np.repeat(sc.reshape(E, K // g, N), g, 1).astype(np.float64)
+    return dev, w, bias.astype(np.float64)
+
+
+def _project(x, ids, w, b):
+    """[A, N] rows x[a]·w[e] + b[e] and the sums of magnitudes (the error scale)."""
+    y = np.zeros((len(ids), w.shape[2]))
+    mag = np.zeros_like(y)
+    for e in np.unique(ids[ids >= 0]).astype(int):
+        r = ids == e
+        y[r] = x[r] @ w[e] + b[e]
+        mag[r] = np.abs(x[r]) @ np.abs(w[e]) + np.abs(b[e])
+    return y, mag
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("xdtype", ["f32", "f16"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_tile_products(bits, xdtype, shape):
+    T, K, N, E, g, k = shape
+    print(f"expert tile int{bits} {xdtype} {shape}", flush=True)
+    route = _route(T, E, k, T + K)
+    ids = route[:, :k].reshape(-1)
+    glu, wg, bg = _weight(E, K, N, g, bits, 11)
+    lin, wl, bl = _weight(E, K, N, g, bits, 23)
+    x = (ref.lcg_f32(T * K, 5) * 2).reshape(T, K)
+    if xdtype == "f16":
+        x = x.astype(np.float16)
+    rd = torch.from_numpy(route).to(DEV)
+    opts = {"bits": bits, "groupSize": g}
+    act = rt.moeUp(torch.from_numpy(x).to(DEV), rd, glu, lin, opts).cpu().numpy()
+    xr = np.repeat(x.astype(np.float64), k, 0)
+    yg, mg = _project(xr, ids, wg, bg)
+    yl, ml = _project(xr, ids, wl, bl)
+    gc, lc = np.minimum(yg, 7.0), np.clip(yl, -7.0, 7.0)
+    want = np.where(ids[:, None] >= 0, gc / (1 + np.exp(-1.702 * gc)) * (lc + 1), 0.0)
+    # Each product's f32 sums are off by at most ~(K/32 + 8)·2^-23 of the sum of
+    # magnitudes, f32 x's two f16 parts by 2^-21 of it; SwiGLU's slopes are below
+    # 1.2·8 (glu) and 7 (lin), its own arithmetic within 2^-20.
+    eps = (K / 32 + 8) * 2.0 ** -23 + 2.0 ** -21
+    np.testing.assert_array_less(np.abs(act - want), 9.6 * eps * mg + 7 * eps * ml
+                                 + 2.0 ** -20 * (1 + np.abs(want)) + 1e-30)
+    # down on plain f32 rows
+    a = (ref.lcg_f32(T * k * K, 9)).reshape(T * k, K)
+    res = ref.lcg_f32(T * N, 4).reshape(T, N)
+    out = rt.moeDown(torch.from_numpy(a).to(DEV), rd, glu, torch.from_numpy(res).to(DEV),
+                     opts).cpu().numpy()
+    y, m = _project(a.astype(np.float64), ids, wg, bg)
+    gates = route[:, k:].astype(np.float64)
+    want = res + (y.reshape(T, k, N) * gates[..., None]).sum(1)
+    mag = np.abs(res) + (m.reshape(T, k, N) * gates[..., None]).sum(1)
+    np.testing.assert_array_less(np.abs(out - want), (eps + (k + 2) * 2.0 ** -23) * mag + 1e-30)
+
+
+def test_int4_f32_range():
+    """int4 weights take f32 x whole: rows near f32's largest and of 1e-20 keep
+    f32's relative error, an infinity or a NaN stays in its row."""
+    T, K, N, E = 40, 128, 64, 2
+    print("expert tile int4 f32 range", flush=True)
+    w, wd, _ = _weight(E, K, N, 32, 4, 3)
+    w.bias = None
+    a = ref.lcg_f32(T * K, 7).reshape(T, K)
+    a[1] *= 1e35
+    a[2] *= 1e-20
+    a[3, 5] = np.inf
+    a[4, 6] = np.nan
+    route = np.zeros((T, 2), np.float32)
+    route[:, 0] = np.arange(T) % E
+    route[:, 1] = 1.0
+    out = rt.moeDown(torch.from_numpy(a).to(DEV), torch.from_numpy(route).to(DEV), w, None,
+                     {"bits": 4, "groupSize": 32}).cpu().numpy()
+    fin = [t for t in range(T) if t not in (3, 4)]
+    for t in fin:
+        want = a[t].astype(np.float64) @ wd[t % E]
+        mag = np.abs(a[t].astype(np.float64)) @ np.abs(wd[t % E])
+        assert np.all(np.abs(out[t] - want) <= 16 * 2.0 ** -23 * mag), t
+    with np.errstate(invalid="ignore"):
+        want = a[3].astype(np.float64) @ wd[1]  # inf · 0 is NaN, else ±inf
+    np.testing.assert_array_equal(np.isnan(out[3]), np.isnan(want))
+    np.testing.assert_array_equal(out[3][~np.isnan(want)], want[~np.isnan(want)])
+    assert np.isnan(out[4]).all()
+
+
+# Layers on each side of the rules: few rows per expert on wide weights, row
+# tiles of 16, 32 and 64, K not a multiple of 32 (I = 1000), and the grouped
+# GEMM's forms from 80 (f16 x: int8 limbs, an odd number of step pairs; f16
+# pairs when I is not a multiple of 64) and 64 (f32 x) rows per expert.
+LAYERS = [MoeConfig("t_wide3", 3, 1024, 16, 4, 2816, "f16"),
+          MoeConfig("t_rows5", 40, 640, 32, 4, 640, "f32"),
+          MoeConfig("t_rows20_i1000", 160, 768, 32, 4, 1000, "f16"),
+          MoeConfig("t_rows40", 320, 640, 32, 4, 640, "f32"),
+          MoeConfig("t_skew", 512, 640, 16, 2, 384, "f16", zipf=1.2, hot_share=0.5, empty=2),
+          MoeConfig("g_limbs_odd", 300, 1024, 6, 2, 1088, "f16"),
+          MoeConfig("g_pairs_i1056", 300, 1024, 6, 2, 1056, "f16"),
+          MoeConfig("g_f32x", 300, 640, 6, 2, 640, "f32")]
+
+
+@pytest.mark.parametrize("cfg", LAYERS, ids=[c.name for c in LAYERS])
+def test_layer_paths(cfg):
+    print(f"layer path {cfg}", flush=True)
+    inp = make_inputs(cfg, seed=12, keep_q=True, bias_rand=True)
+    inp.residual.copy_(torch.randn(tuple(inp.residual.shape), generator=torch.Generator().manual_seed(6)))
+    out, route = rt.moe_layer(inp.x, inp.router_w, inp.router_b, inp.glu, inp.lin, inp.down,
+                              inp.residual, cfg.k, return_route=True)
+    x = inp.x.float().cpu().numpy()
+    want_route = ref.topk(ref.router_logits(x, inp.router_w.cpu().numpy(),
+                                            inp.router_b.cpu().numpy()), cfg.k)
+    w = {n: (ref.pack_ekn(inp.q[n].numpy(), 8), getattr(inp, n).scales.cpu().numpy(),
+             getattr(inp, n).bias.cpu().numpy()) for n in ("glu", "lin", "down")}
+    act = ref.moe_up(x, want_route, w["glu"], w["lin"], 8, cfg.d, cfg.E)
+    want = ref.moe_down(act, want_route, w["down"], inp.residual.cpu().numpy(), 8, cfg.I, cfg.E)
+    assert np.array_equal(route.cpu().numpy()[:, :cfg.k], want_route[:, :cfg.k])
+    assert_close(out.cpu().numpy(), want, what=cfg.name)
