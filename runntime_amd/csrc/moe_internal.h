@@ -94,11 +94,18 @@ constexpr int DISPATCH_MAX_E = 1024;
 // Device-side bookkeeping written by the dispatch scan (int32 each).
 enum MetaSlot { META_VALID = 0, META_ACTIVE = 1, META_MAXCNT = 2, META_TILES = 3, META_N = 8 };
 
-// Largest token count whose routing and dispatch one block does (fused).
+// Largest token count of the router's small chunk kernel without a dispatch.
 constexpr int SMALL_T = 16;
-// Calls up to FUSED_T tokens (T·k ≤ FUSED_T·MAX_K) run the router's fold,
-// top-k and dispatch in one block per call.
+// Calls up to FUSED_T tokens: the router's small chunk kernel, which can
+// normalise x while staging it.
 constexpr int FUSED_T = 64;
+// Calls up to FUSED_A assignments run the router's fold, top-k and dispatch in
+// one block per call; above, a wavefront per token over many blocks and the
+// one-block sort are faster (whole layer with 128-column experts, fused and
+// split, µs: E 128 top-4, 12 tokens 33.1, 33.6; 16 tokens 35.8, 35.1; 64
+// tokens 49.6, 34.1; E 64 top-8, d 2048, 8 tokens 43.8, 43.4, 64 tokens 78.7,
+// 49.5; E 8 top-2, 16 tokens 25.4, 26.1, 64 tokens 33.0, 26.5).
+constexpr int FUSED_A = 48;
 // Rows per M-tile of the grouped GEMM; the dispatch counts M-tiles with it.
 constexpr int GEMM_TILE_M = 128;
 
@@ -158,8 +165,8 @@ struct RouterArgs {
   // up product's prologue (ExpertArgs::fr_partial).
   int chunks_only;
 };
-// Router + top-k. With T <= FUSED_T and `db` given, the dispatch of each call
-// is built in the same kernel and `dispatched` is set.
+// Router + top-k. With T·k <= FUSED_A and `db` given, the dispatch of each
+// call is built in the same kernel and `dispatched` is set.
 int launch_router_topk(const RouterArgs &ra, const DispatchBufs *db, int tile_m, bool *dispatched,
                        hipStream_t s);
 int launch_dispatch(const float *route, int64_t route_cs, int T, int E, int k, int calls,

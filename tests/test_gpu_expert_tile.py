@@ -152,3 +152,21 @@ def test_layer_paths(cfg):
     want = ref.moe_down(act, want_route, w["down"], inp.residual.cpu().numpy(), 8, cfg.I, cfg.E)
     assert np.array_equal(route.cpu().numpy()[:, :cfg.k], want_route[:, :cfg.k])
     assert_close(out.cpu().numpy(), want, what=cfg.name)
+
+
+# Dispatch over the routes of each sort kernel: one block (1, 2, 4 and 8
+# chunks a wavefront, runs that end inside a chunk), three kernels above 8192
+# assignments or 512 experts; ids that name no expert leave -1 at the end.
+@pytest.mark.parametrize("T,k,E", [(1, 1, 1), (63, 1, 5), (77, 4, 128), (257, 4, 130), (683, 3, 64),
+                                   (1025, 4, 512), (1365, 6, 33), (2048, 4, 128), (2049, 4, 128),
+                                   (40, 2, 700)])
+def test_dispatch_one_block(T, k, E):
+    print(f"dispatch T={T} k={k} E={E}", flush=True)
+    rng = np.random.default_rng(T)
+    route = np.ones((T, 2 * k), np.float32)
+    route[:, :k] = rng.integers(0, E, (T, k))
+    route[::5, 0] = rng.choice([-1.0, E, 0.5, np.nan], len(route[::5]))
+    perm, off = rt.dispatch(torch.from_numpy(route).to(DEV), E)
+    want_perm, _, want_off = ref.dispatch(route, E)
+    np.testing.assert_array_equal(off.cpu().numpy(), want_off)
+    np.testing.assert_array_equal(perm.cpu().numpy(), want_perm)
