@@ -170,3 +170,22 @@ def test_dispatch_one_block(T, k, E):
     want_perm, _, want_off = ref.dispatch(route, E)
     np.testing.assert_array_equal(off.cpu().numpy(), want_off)
     np.testing.assert_array_equal(perm.cpu().numpy(), want_perm)
+
+
+@pytest.mark.parametrize("E,k", [(7, 3), (64, 8), (130, 4), (513, 16)])
+def test_topk_special_logits(E, k):
+    """Infinities, NaN, both zeros (equal, the lower id first), values at and
+    below the −3.4e38 start, and rows with fewer candidates than k."""
+    print(f"topk special E={E} k={k}", flush=True)
+    rng = np.random.default_rng(E)
+    x = rng.choice(np.array([np.inf, -np.inf, np.nan, 0.0, -0.0, -3.4e38, -3.3e38, 1.5, -1.5,
+                             1e-40, -1e-40], np.float32), (40, E))
+    x[5] = -np.inf
+    x[6] = np.nan
+    x[7, 1:] = -np.inf
+    x[8] = np.where(np.arange(E) % 2, 0.0, -0.0)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = ref.topk(x, k)
+    got = rt.topk(torch.from_numpy(x).to(DEV), k).cpu().numpy()
+    np.testing.assert_array_equal(got[:, :k], want[:, :k])
+    np.testing.assert_allclose(got[:, k:], want[:, k:], atol=1e-7, rtol=1e-5, equal_nan=True)
