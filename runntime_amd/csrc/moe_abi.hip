@@ -955,9 +955,7 @@ extern "C" int moe_linear(moe_ctx *ctx, const float *x, const float *w, const fl
   if (rc) return rc;
   REQUIRE(T >= 1 && K >= 1 && N >= 1, "linear: T, K and N must be positive");
   REQUIRE(x && w && out, "linear: NULL tensor");
-  if ((rc = moe_ws_ensure(ctx, linear_ws_bytes(T, K, N)))) return rc;
-  if ((rc = launch_linear(x, w, bias, addend, out, (float *)ctx->ws, T, K, N, ctx->stream)))
-    return rc;
+  if ((rc = launch_linear(x, w, bias, addend, out, T, K, N, ctx->stream))) return rc;
   return after_launch("linear");
 }
 
