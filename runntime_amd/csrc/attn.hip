@@ -22,6 +22,8 @@
 
 #include <math.h>
 
+#include <algorithm>
+#include <initializer_list>
 #include <type_traits>
 
 namespace {
@@ -308,6 +310,280 @@ __global__ __launch_bounds__(AW *WAVE) void k_sdpa(AttnArgs a) {
   }
 }
 
+// ------------------------------------------------ on the f32 matrix cores
+//
+// k_sdpa_mfma (head_dim 64 or 128): a wavefront takes 16 query rows of one
+// head and walks its keys 16·NT at a time with v_mfma_f32_16x16x4_f32 (f32
+// operands and sums):
+//   Sᵀ = K·Qᵀ  keys × rows: lane (r = lane mod 16, g = lane / 16) gets row r's
+//              scores of keys 4g .. 4g + 3 of each 16,
+//   Oᵀ = Vᵀ·Pᵀ head columns × rows: its B operand is exactly those values, so P
+//              never leaves the lane's registers.
+// A lane keeps one row's running max and sum (its four lanes hold equal
+// copies; two exchanges across them per step). Operands come from memory in
+// 16-byte loads, four consecutive head columns a lane: step (s, j) of Sᵀ uses
+// element j of columns 16s + 4g .. + 3 of K and Q; step j of Oᵀ key 4g + j, its
+// column tile c of slab b the columns 64b + 4·(lane mod 16) + c. Nothing is
+// staged in LDS; the wavefronts of a block (HW heads of one kv head) walk the
+// same keys together, so K, V and the rope tables come out of L1.
+// KS > 1 splits the keys of a head over KS wavefronts, whose sums meet in LDS
+// in order (short sequences, few heads).
+// Bound by latency and L1 (each wavefront reads K, V and the rope tables of
+// its keys, 32 KB a step). Against k_sdpa below (f32 VALU, K and V through
+// LDS), 14 heads over 2 kv heads of 64, rope, window ±128: 64 rows 11.4 → 7.5
+// µs, 1500 rows 126 → 51 (27 TFLOP/s), 4096 rows 280 → 78.
+template <typename T> struct Ld4;
+template <> struct Ld4<float> {
+  static __device__ __forceinline__ float4 at(const float *p) { return *(const float4 *)p; }
+};
+template <> struct Ld4<_Float16> {
+  static __device__ __forceinline__ float4 at(const _Float16 *p) {
+    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+    const h4 v = *(const h4 *)p;
+    return make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
+  }
+};
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ void st4(float *p, float x, float y, float z, float w) {
+  *(float4 *)p = make_float4(x, y, z, w);
+}
+__device__ __forceinline__ void st4(_Float16 *p, float x, float y, float z, float w) {
+  typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+  *(h4 *)p = h4{(_Float16)x, (_Float16)y, (_Float16)z, (_Float16)w};
+}
+
+// Four head columns after rope: two interleaved pairs (the expression of
+// `roped`).
+__device__ __forceinline__ floatx4 rope4(float4 x, float4 c, float4 s) {
+  return floatx4{x.x * c.x - x.y * s.x, x.y * c.y + x.x * s.y, x.z * c.z - x.w * s.z,
+                 x.w * c.w + x.z * s.w};
+}
+
+template <typename T, int NB, int NT, bool ROPE>  // head_dim 64·NB, 16·NT keys a step
+__global__ __launch_bounds__(512) void k_sdpa_mfma(AttnArgs a, int hw, int ksplit) {
+  constexpr int HD = 64 * NB, NS = HD / 16;
+  constexpr int KC = 16 * NT;
+  extern __shared__ __align__(16) float mlds[];
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wave = threadIdx.x / WAVE;
+  const int part = wave / hw;
+  const int G = a.q_heads / a.kv_heads;
+  const int hgroups = (G + hw - 1) / hw;
+  const int kvh = blockIdx.y / hgroups;
+  const int hg = (blockIdx.y - kvh * hgroups) * hw + wave % hw;
+  const bool head_ok = hg < G;
+  const int h = kvh * G + (head_ok ? hg : 0);
+  const int m = lane & 15, g = lane >> 4;
+  const int row0 = blockIdx.x * 16;
+  const int row = min(row0 + m, a.q_len - 1);
+  const T *kp = (const T *)a.k + (int64_t)kvh * HD;
+  const T *vp = (const T *)a.v + (int64_t)kvh * HD;
+
+  // The row's keys, and the tile's.
+  int lo, hi;
+  {
+    const long long qpos = (long long)a.q_pos_offset + row;
+    long long l = a.window_left < 0 ? 0 : qpos - a.window_left;
+    long long u = a.window_right < 0 ? (long long)a.kv_len - 1 : qpos + a.window_right;
+    if (l < 0) l = 0;
+    if (u > a.kv_len - 1) u = a.kv_len - 1;
+    if (a.segs) {
+      const long long s0 = (long long)a.segs[2 * row], s1 = (long long)a.segs[2 * row + 1] - 1;
+      if (s0 > l) l = s0;
+      if (s1 < u) u = s1;
+    }
+    lo = (int)l;
+    hi = (int)(u < l - 1 ? l - 1 : u);  // empty: hi < lo
+  }
+  int blo = hi >= lo ? lo : 0x7fffffff, bhi = hi >= lo ? hi : -1;
+#pragma unroll
+  for (int x = 1; x < 16; x <<= 1) {
+    blo = min(blo, __shfl_xor(blo, x));
+    bhi = max(bhi, __shfl_xor(bhi, x));
+  }
+  blo = __builtin_amdgcn_readfirstlane(blo);
+  bhi = __builtin_amdgcn_readfirstlane(bhi);
+  // This wavefront's steps of KC keys: an equal run of them per part.
+  const int nstep = bhi >= blo ? (bhi - blo) / KC + 1 : 0;
+  const int per = (nstep + ksplit - 1) / ksplit;
+  const int c_first = part * per, c_last = min(nstep, c_first + per);
+
+  floatx4 q[NS];
+#pragma unroll
+  for (int s = 0; s < NS; s++) {
+    const int x = 16 * s + 4 * g;
+    const float4 v = Ld4<T>::at((const T *)a.q + (int64_t)row * a.q_rs + (int64_t)h * HD + x);
+    if constexpr (ROPE)
+      q[s] = rope4(v, *(const float4 *)(a.rope_cos + (int64_t)row * HD + x),
+                   *(const float4 *)(a.rope_sin + (int64_t)row * HD + x));
+    else
+      q[s] = floatx4{v.x, v.y, v.z, v.w};
+  }
+  struct KTile {
+    float4 k[NT][NS], c[ROPE ? NT : 1][ROPE ? NS : 1], s[ROPE ? NT : 1][ROPE ? NS : 1];
+  };
+  // Keys past the tile's last read that one (their probability is 0).
+  auto load_k = [&](int step, KTile &t) {
+#pragma unroll
+    for (int n = 0; n < NT; n++) {
+      const int64_t key = min(blo + step * KC + 16 * n + m, bhi);
+#pragma unroll
+      for (int s = 0; s < NS; s++) {
+        const int x = 16 * s + 4 * g;
+        t.k[n][s] = Ld4<T>::at(kp + key * a.k_rs + x);
+        if constexpr (ROPE) {
+          t.c[n][s] = *(const float4 *)(a.rope_cos + key * HD + x);
+          t.s[n][s] = *(const float4 *)(a.rope_sin + key * HD + x);
+        }
+      }
+    }
+  };
+  float4 v[NT][4][NB];
+  auto load_v = [&](int step) {
+#pragma unroll
+    for (int n = 0; n < NT; n++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int64_t key = min(blo + step * KC + 16 * n + 4 * g + j, bhi);
+#pragma unroll
+        for (int b = 0; b < NB; b++) v[n][j][b] = Ld4<T>::at(vp + key * a.v_rs + 64 * b + 4 * m);
+      }
+  };
+  float mx = -INFINITY, sum = 0.f;
+  floatx4 acc[NB][4];
+#pragma unroll
+  for (int b = 0; b < NB; b++)
+#pragma unroll
+    for (int c = 0; c < 4; c++) acc[b][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+  if (c_first < c_last) {  // then blo ≤ bhi: every address is a key's
+    KTile kt;
+    load_k(c_first, kt);
+    load_v(c_first);
+    for (int st = c_first; st < c_last; st++) {
+      floatx4 sc[NT];
+#pragma unroll
+      for (int n = 0; n < NT; n++) {
+        // two chains: halves the dependent MFMA latency
+        floatx4 s0 = floatx4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+          floatx4 k4;
+          if constexpr (ROPE)
+            k4 = rope4(kt.k[n][s], kt.c[n][s], kt.s[n][s]);
+          else
+            k4 = floatx4{kt.k[n][s].x, kt.k[n][s].y, kt.k[n][s].z, kt.k[n][s].w};
+          s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[0], q[s][0], s0, 0, 0, 0);
+          s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[1], q[s][1], s1, 0, 0, 0);
+          s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[2], q[s][2], s0, 0, 0, 0);
+          s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[3], q[s][3], s1, 0, 0, 0);
+        }
+        sc[n] = s0 + s1;
+      }
+      load_k(min(st + 1, c_last - 1), kt);  // lands under the softmax and P·V
+      const int key0 = blo + st * KC + 4 * g;
+      float top = -INFINITY;
+#pragma unroll
+      for (int n = 0; n < NT; n++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const int key = key0 + 16 * n + j;
+          float x = sc[n][j];
+          if (a.has_kb && key >= a.kb_start && key < a.kb_end) x += a.kb_value;
+          x = key >= lo && key <= hi ? x : -INFINITY;
+          sc[n][j] = x;
+          top = fmaxf(top, x);
+        }
+      top = fmaxf(top, __shfl_xor(top, 16));
+      top = fmaxf(top, __shfl_xor(top, 32));
+      const float mn = fmaxf(mx, top);
+      const float base = mn == -INFINITY ? 0.f : mn;  // nothing seen yet
+      const float scale = mx == -INFINITY ? 0.f : expf(mx - base);
+      float add = 0.f;
+#pragma unroll
+      for (int n = 0; n < NT; n++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const int key = key0 + 16 * n + j;
+          const float p = key >= lo && key <= hi ? expf(sc[n][j] - base) : 0.f;
+          sc[n][j] = p;
+          add += p;
+        }
+      add += __shfl_xor(add, 16);
+      add += __shfl_xor(add, 32);
+      sum = sum * scale + add;
+      mx = mn;
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          floatx4 o = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int n = 0; n < NT; n++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+              const float4 &vv = v[n][j][b];
+              const float ve = c == 0 ? vv.x : c == 1 ? vv.y : c == 2 ? vv.z : vv.w;
+              o = __builtin_amdgcn_mfma_f32_16x16x4f32(ve, sc[n][j], o, 0, 0, 0);
+            }
+          acc[b][c] = acc[b][c] * scale + o;
+        }
+      load_v(min(st + 1, c_last - 1));
+    }
+  }
+  // acc[b][c][i]: row `row`, head column 64b + 16g + 4i + c.
+  if (ksplit > 1) {
+    // The later parts leave (max, sum, acc); the first folds them in, in order.
+    constexpr int SLOT = (2 + 16 * NB) * WAVE;
+    if (part > 0) {
+      float *d = mlds + ((part - 1) * hw + wave % hw) * SLOT + lane;
+      d[0] = mx;
+      d[WAVE] = sum;
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) d[(2 + 16 * b + 4 * c + i) * WAVE] = acc[b][c][i];
+    }
+    __syncthreads();
+    if (part > 0) return;
+    for (int p = 1; p < ksplit; p++) {
+      const float *d = mlds + ((p - 1) * hw + wave % hw) * SLOT + lane;
+      const float m2 = d[0];
+      const float mn = fmaxf(mx, m2);
+      const float base = mn == -INFINITY ? 0.f : mn;
+      const float f1 = mx == -INFINITY ? 0.f : expf(mx - base);
+      const float f2 = m2 == -INFINITY ? 0.f : expf(m2 - base);
+      sum = sum * f1 + d[WAVE] * f2;
+      mx = mn;
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            acc[b][c][i] = acc[b][c][i] * f1 + d[(2 + 16 * b + 4 * c + i) * WAVE] * f2;
+    }
+  }
+  if (!head_ok || row0 + m >= a.q_len) return;
+  // Sinks join the denominator; store.
+  const float sg = a.sinks ? a.sinks[h] * LN2 : -INFINITY;
+  const float mf = fmaxf(mx, sg);
+  float f = 0.f;
+  if (mf != -INFINITY) {
+    const float scale = mx == -INFINITY ? 0.f : expf(mx - mf);
+    f = scale * (1.0f / (sum * scale + (a.sinks ? expf(sg - mf) : 0.f)));
+  }
+  T *out = (T *)a.out + (int64_t)row * a.o_rs + (int64_t)h * HD + 16 * g;
+#pragma unroll
+  for (int b = 0; b < NB; b++)
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      st4(out + 64 * b + 4 * i, acc[b][0][i] * f, acc[b][1][i] * f, acc[b][2][i] * f,
+          acc[b][3][i] * f);
+}
+
 }  // namespace
 
 int launch_rope(const void *x, moe_dtype dt, int rows, int cols, int hd, int src_start, int width,
@@ -329,6 +605,17 @@ int launch_rope(const void *x, moe_dtype dt, int rows, int cols, int hd, int src
   return 0;
 }
 
+// k_sdpa_mfma: head_dim 64 or 128, every row's four-column groups aligned.
+static bool sdpa_mfma_ok(const AttnArgs &a) {
+  if (a.head_dim != 64 && a.head_dim != 128) return false;
+  const uintptr_t al = a.dtype == MOE_F16 ? 8 : 16;
+  for (const void *p : {a.q, a.k, a.v, (const void *)a.out})
+    if ((uintptr_t)p % al) return false;
+  if (a.q_rs % 4 || a.k_rs % 4 || a.v_rs % 4 || a.o_rs % 4) return false;
+  return (uintptr_t)a.rope_cos % 16 == 0 && (uintptr_t)a.rope_sin % 16 == 0 &&
+         (int64_t)a.kv_heads * (a.q_heads / a.kv_heads) <= 65535;
+}
+
 int launch_sdpa(AttnArgs a, hipStream_t s) {
   MOE_NONNULL(a.q);
   MOE_NONNULL(a.k);
@@ -338,6 +625,41 @@ int launch_sdpa(AttnArgs a, hipStream_t s) {
   if (G > AW * AI)
     return moe_fail(MOE_INVALID_ARGUMENT, "sdpa: more than " + std::to_string(AW * AI) +
                                               " query heads per kv head");
+  if (sdpa_mfma_ok(a)) {
+    // Keys of a row tile: the window and 15 more rows, at most kv_len.
+    const int64_t span = a.window_left < 0 || a.window_right < 0
+                             ? a.kv_len
+                             : std::min((int64_t)a.kv_len, (int64_t)(a.window_left + a.window_right + 16));
+    const int kc = a.head_dim == 64 ? 32 : 16;
+    const int64_t nstep = (span + kc - 1) / kc;
+    const int64_t tiles = ((int64_t)a.q_len + 15) / 16;
+    // Heads of a kv head together (K, V and rope tables from one L1) once that
+    // gives two blocks a CU, else a block per head; up to 4 wavefronts over its
+    // keys while heads × row tiles × parts stay near 2500 (attention block,
+    // µs, one head and 1, 2, 4, 8 parts, seven heads: 300 rows 58, 50, 46, 51,
+    // 81; 1500 rows 109, 109, 113, 131, 115; 4096 rows 259, 244, 250, 298, 236).
+    const int64_t heads = tiles * a.q_heads;
+    int hw = std::min(G, 8);
+    if (tiles * a.kv_heads * ((G + hw - 1) / hw) < 512) hw = 1;
+    int ks = 1;
+    while (hw == 1 && ks < 4 && ks * 2 <= nstep && heads * ks * 2 <= 2700) ks *= 2;
+    const dim3 grid((unsigned)tiles, a.kv_heads * ((G + hw - 1) / hw)), block(WAVE * hw * ks);
+    const size_t lds = (size_t)(ks - 1) * hw * (2 + 16 * (a.head_dim / 64)) * WAVE * 4;
+#define SDPA_M(T_, NB_, NT_)                                                                     \
+  do {                                                                                           \
+    if (a.rope_cos) hipLaunchKernelGGL((k_sdpa_mfma<T_, NB_, NT_, true>), grid, block, lds, s, a, hw, ks); \
+    else hipLaunchKernelGGL((k_sdpa_mfma<T_, NB_, NT_, false>), grid, block, lds, s, a, hw, ks); \
+  } while (0)
+    if (a.dtype == MOE_F16) {
+      if (a.head_dim == 64) SDPA_M(_Float16, 1, 2);
+      else SDPA_M(_Float16, 2, 1);
+    } else {
+      if (a.head_dim == 64) SDPA_M(float, 1, 2);
+      else SDPA_M(float, 2, 1);
+    }
+#undef SDPA_M
+    return 0;
+  }
   // Rows per block: up to the 64 items a block holds, fewer for short
   // sequences so that the grid still has ~512 blocks (each block stages its
   // keys once; more rows per block share more of them).
