@@ -8,19 +8,33 @@
 // SwiGLU, the out gather, gate-weighted sum over the slots, + x).
 //
 // Rows arrive grouped by expert (dispatch.hip), so each expert's weight
-// rows stream once per chunk of its rows, where the reference reads them
-// once per (row, slot). The weights are row-major [K, N] per expert: a
-// lane owns 4 consecutive columns (one 8- or 16-byte load per weight row,
-// 64 lanes reading one contiguous stretch), and the block's 4 wavefronts
-// split K; their partial sums meet in LDS, added in wavefront order. The
-// arithmetic is f32 VALU fma: at decode sizes the kernel streams weights,
-// and MFMA would need the weights transposed first.
+// rows stream once per 16·RT of its rows, where the reference reads them
+// once per (row, slot). A block is one row tile × 64 columns; its 8
+// wavefronts split K (up: four parts of glu and four of lin), and their sums
+// meet in LDS, added in part order, before the bias and the SwiGLU. The
+// products are v_mfma_f32_16x16x4_f32: the weights are row-major [K, N], so
+// per 16 k a lane loads four consecutive columns of four weight rows (whole
+// 256-byte runs per 16 lanes, read once: nontemporal) and four consecutive k
+// of its row, and MFMA step j takes weight row j and element j, with no LDS
+// or conversion between (f16 values widen to f32 first). FPD steps are in
+// flight per wavefront. A step's sums start from zero and join the total, so
+// no chain of additions is longer than 16 or K / 64 terms.
+//
+// Bound by the weight stream. Measured (E 128, top-4, 640 × 640, 77 tokens,
+// f32 weights) against 4-row chunks on the VALU with x in LDS: up 112 → 63 µs,
+// down 66 → 34 (6.1 and 5.6 TB/s); 500 tokens, whole block, 649 → 171, f16
+// 505 → 126. More steps in flight cost wavefronts that fit (77 tokens, one to
+// four steps: 123, 133, 151, 167 µs a block).
 #include "moe_internal.h"
 
 namespace {
 
 constexpr int WAVE = 64;
-constexpr int FCOLS = 4 * WAVE;  // columns per block
+constexpr int FWAVES = 8;
+constexpr int FSTEP = 16;  // k per step
+constexpr int FCOLS = 64;  // columns per block
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float swiglu(float glu, float lin) {
   // activations.ts:127-133, exp via the hardware 2^x and the quotient via
@@ -31,130 +45,192 @@ __device__ __forceinline__ float swiglu(float glu, float lin) {
   return g * __builtin_amdgcn_rcpf(1.0f + e) * (l + 1.0f);
 }
 
-__device__ __forceinline__ float4 load4w(const float *p) { return *(const float4 *)p; }
-__device__ __forceinline__ float4 load4w(const _Float16 *p) {
-  typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-  const h4 v = *(const h4 *)p;
-  return make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
+// Weights are read once: nontemporal buffer loads. A step's 16 weight rows get
+// a descriptor of their own (scalar arithmetic), so the lanes' offsets are
+// loop constants and a row past K or a column past N reads zeros. (64-bit row
+// addresses per lane cost more VALU time than the products.)
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+constexpr uint32_t F_OOB = 0x80000000u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const void *base, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, bytes, 0x00020000 /* raw, 32-bit */);
 }
-__device__ __forceinline__ void store4(float *p, float4 v) { *(float4 *)p = v; }
-__device__ __forceinline__ void store4(_Float16 *p, float4 v) {
-  typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-  *(h4 *)p = h4{(_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
+__device__ __forceinline__ void stream4(floatx4 &d, __amdgpu_buffer_rsrc_t r, uint32_t off) {
+  d = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 2 /* nt */));
 }
-__device__ __forceinline__ float4 fma4(float a, float4 w, float4 c) {
-  return make_float4(fmaf(a, w.x, c.x), fmaf(a, w.y, c.y), fmaf(a, w.z, c.z), fmaf(a, w.w, c.w));
+__device__ __forceinline__ void stream4(half4 &d, __amdgpu_buffer_rsrc_t r, uint32_t off) {
+  d = __builtin_bit_cast(half4, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 2 /* nt */));
 }
-__device__ __forceinline__ float4 add4(float4 a, float4 b) {
-  return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+__device__ __forceinline__ floatx4 load4(const float *p) { return *(const floatx4 *)p; }
+__device__ __forceinline__ half4 load4(const _Float16 *p) { return *(const half4 *)p; }
+__device__ __forceinline__ floatx4 wide(floatx4 v) { return v; }
+__device__ __forceinline__ floatx4 wide(half4 v) {
+  return floatx4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
 }
+__device__ __forceinline__ void store4(float *p, floatx4 v) { *(floatx4 *)p = v; }
+__device__ __forceinline__ void store4(_Float16 *p, floatx4 v) {
+  *(half4 *)p = half4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+}
+template <typename T> struct Vec4;
+template <> struct Vec4<float> { typedef floatx4 type; };
+template <> struct Vec4<_Float16> { typedef half4 type; };
 
 // MODE_UP: act[a] = swiglu(x·glu[e] + bias_glu[e], x·lin[e] + bias_lin[e]).
 // MODE_DOWN (and the plain gather): out[a] = x·w[e] + bias[e].
 // AT: activation type, WT: weight and bias type, OT: output type.
-// FW wavefronts split K; FRC rows per chunk. Decode (experts with a row or
-// two) runs 8 × 2: twice the wavefronts and loads in flight of 4 × 4, whose
-// larger chunks suit experts with more rows (fewer passes over the weights).
-// FU weight rows per loop iteration are in flight: 8 with 2 rows per chunk,
-// 4 with 4 (where 8 costs more registers than it gains).
-template <int MODE, typename AT, typename WT, typename OT, int FW, int FRC, int FU>
-__global__ __launch_bounds__(FW * WAVE) void k_float_expert(FloatArgs p) {
+enum KForm { K_STEPS = 0, K_QUADS = 1, K_ANY = 2 };  // K % 16 == 0, % 4 == 0 (rows of a aligned), any
+// FPD: steps loaded (the one multiplied and those ahead of it).
+template <int MODE, typename AT, typename WT, typename OT, int RT, int KF, int FPD>
+__global__ __launch_bounds__(FWAVES *WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_float_tile(FloatArgs p, int gx) {
   constexpr int NS = MODE == MODE_UP ? 2 : 1;
-  extern __shared__ __align__(16) unsigned char smem[];
-  float *xs = (float *)smem;                                  // [FRC][K]
-  float4 *red = (float4 *)(smem + (size_t)FRC * p.K * 4);     // [FW][NS][FRC][WAVE]
+  constexpr int KW = FWAVES / NS;           // wavefronts per weight array
+  constexpr int ROWS = 16 * RT;
+  typedef typename Vec4<AT>::type av4;
+  typedef typename Vec4<WT>::type wv4;
+  __shared__ floatx4 red[FWAVES][4 * RT][WAVE];
 
-  const int call = blockIdx.z;
-  const int4 desc = ((const int4 *)(p.db.active + call * p.db.act_cs()))[blockIdx.y];
-  const int e = desc.x;
-  if (e < 0) return;
-  const int p0 = desc.y, cnt = desc.z;
-  const int32_t *perm = p.db.perm + call * p.db.perm_cs();
-  const AT *abase = (const AT *)p.a + call * p.a_cs;
-  OT *out = (OT *)p.out + call * p.out_cs;
-  const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
-  const int c0 = blockIdx.x * FCOLS + 4 * lane;
-  const bool col_ok = c0 < p.N;
-  const int kq = (p.K + FW - 1) / FW;
-  const int kb = wave * kq, ke = min(p.K, kb + kq);
-  const WT *w[NS];
-  const WT *b[NS];
-#pragma unroll
-  for (int s = 0; s < NS; s++) {
-    w[s] = (const WT *)(s == 0 ? p.w0 : p.w1) + call * (s == 0 ? p.w0_cs : p.w1_cs) +
-           (int64_t)e * p.K * p.N + (col_ok ? c0 : 0);
-    const WT *bb = (const WT *)(s == 0 ? p.b0 : p.b1);
-    b[s] = bb ? bb + call * (s == 0 ? p.b0_cs : p.b1_cs) + (int64_t)e * p.N + (col_ok ? c0 : 0)
-              : nullptr;
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int call = blockIdx.y;
+  // This block's row tile and column block, one contiguous range of the
+  // call's tiles per XCD (blocks go round-robin over the 8 XCDs).
+  const int32_t *meta = p.db.meta + call * p.db.meta_cs();
+  const int4 *active = (const int4 *)(p.db.active + call * p.db.act_cs());
+  const int E = p.db.E;
+  int4 ad = active[min(lane, E - 1)];
+  const int na = meta[META_ACTIVE];
+  const int total = meta[META_TILES] * gx;
+  const int per = (total + 7) / 8;
+  const int slot = blockIdx.x >> 3;
+  const int o = (blockIdx.x & 7) * per + slot;
+  if (slot >= per || o >= total) return;
+  const int mt = o / gx, xb = o - mt * gx;
+  int hit = __popcll(__ballot(lane < na && ad.w <= mt)) - 1;
+  for (int b = WAVE; hit == WAVE - 1 && b < na; b += WAVE) {
+    const int4 nx = active[min(b + lane, na - 1)];
+    const int h = __popcll(__ballot(b + lane < na && nx.w <= mt)) - 1;
+    if (h < 0) break;
+    ad = nx;
+    hit = h;
   }
+  const int e = __builtin_amdgcn_readlane(ad.x, hit);
+  const int r0 = (mt - __builtin_amdgcn_readlane(ad.w, hit)) * ROWS;
+  const int rows = min(ROWS, __builtin_amdgcn_readlane(ad.z, hit) - r0);
+  const int p0 = __builtin_amdgcn_readlane(ad.y, hit) + r0;
+  const int32_t *perm = p.db.perm + call * p.db.perm_cs() + p0;
 
-  for (int r0 = 0; r0 < cnt; r0 += FRC) {
-    const int rows = min(FRC, cnt - r0);
-    for (int i = threadIdx.x; i < FRC * p.K; i += FW * WAVE) {
-      const int r = i / p.K, kk = i - r * p.K;
-      float v = 0.f;
-      if (r < rows) v = (float)abase[(int64_t)(perm[p0 + r0 + r] / p.a_row_div) * p.K + kk];
-      xs[i] = v;
-    }
-    __syncthreads();
-    float4 acc[NS][FRC];
+  const int arr = wave / KW, part = wave % KW;
+  const int m = lane & 15, kq = lane >> 4;
+  const int col = xb * FCOLS + 4 * m;  // N is a multiple of 4
+  const bool col_ok = col < p.N;
+  const int64_t wcall = call * (arr ? p.w1_cs : p.w0_cs);
+  const WT *w = (const WT *)(arr ? p.w1 : p.w0) + wcall + (int64_t)e * p.K * p.N;
+  uint32_t woff[4];
 #pragma unroll
-    for (int s = 0; s < NS; s++)
+  for (int j = 0; j < 4; j++)
+    woff[j] = col_ok ? ((uint32_t)(4 * kq + j) * (uint32_t)p.N + col) * (uint32_t)sizeof(WT) : F_OOB;
+  // Rows past the tile read its first one; their sums are not stored.
+  const AT *xr[RT];
 #pragma unroll
-      for (int r = 0; r < FRC; r++) acc[s][r] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (col_ok) {
-      // FU weight rows per iteration, every load issued before the fmas.
-      int kk = kb;
-      for (; kk + FU <= ke; kk += FU) {
-        float4 wv[NS][FU];
+  for (int t = 0; t < RT; t++) {
+    const int r = 16 * t + m;
+    xr[t] = (const AT *)p.a + call * p.a_cs +
+            (int64_t)(perm[r < rows ? r : 0] / p.a_row_div) * p.K;
+  }
+  const int steps = (p.K + FSTEP - 1) / FSTEP;
+  const int sp = (steps + KW - 1) / KW;
+  const int s0 = part * sp, s1 = min(steps, s0 + sp);
+
+  struct Step {
+    av4 a[RT];
+    wv4 b[4];
+  };
+  // Addresses of a stay inside its rows: a step past the last reads that one
+  // (not used), a k past K reads k = 0.
+  auto load = [&](int s, Step &d) {
+    s = min(s, steps - 1);
+    const int k = s * FSTEP + 4 * kq;
+    const int left = KF == K_STEPS ? FSTEP : min(FSTEP, p.K - s * FSTEP);
+    const __amdgpu_buffer_rsrc_t wr =
+        rows_rsrc(w + (int64_t)s * FSTEP * p.N, left * p.N * (int)sizeof(WT));
 #pragma unroll
-        for (int s = 0; s < NS; s++)
+    for (int j = 0; j < 4; j++) stream4(d.b[j], wr, woff[j]);
 #pragma unroll
-          for (int u = 0; u < FU; u++) wv[s][u] = load4w(w[s] + (int64_t)(kk + u) * p.N);
+    for (int t = 0; t < RT; t++) {
+      if constexpr (KF != K_ANY) {
+        d.a[t] = load4(xr[t] + (KF == K_STEPS || k < p.K ? k : 0));
+      } else {
 #pragma unroll
-        for (int u = 0; u < FU; u++)
-#pragma unroll
-          for (int r = 0; r < FRC; r++) {
-            const float xv = xs[r * p.K + kk + u];
-#pragma unroll
-            for (int s = 0; s < NS; s++) acc[s][r] = fma4(xv, wv[s][u], acc[s][r]);
-          }
-      }
-      for (; kk < ke; kk++) {
-#pragma unroll
-        for (int s = 0; s < NS; s++) {
-          const float4 wv = load4w(w[s] + (int64_t)kk * p.N);
-#pragma unroll
-          for (int r = 0; r < FRC; r++) acc[s][r] = fma4(xs[r * p.K + kk], wv, acc[s][r]);
-        }
-      }
-    }
-#pragma unroll
-    for (int s = 0; s < NS; s++)
-#pragma unroll
-      for (int r = 0; r < FRC; r++) red[((wave * NS + s) * FRC + r) * WAVE + lane] = acc[s][r];
-    __syncthreads();
-    // Wavefront 0 adds the K quarters in order, then the bias and (up) the
-    // SwiGLU, and writes each row.
-    if (wave == 0 && col_ok) {
-      for (int r = 0; r < rows; r++) {
-        float4 v[NS];
-#pragma unroll
-        for (int s = 0; s < NS; s++) {
-          float4 t = red[((0 * NS + s) * FRC + r) * WAVE + lane];
-#pragma unroll
-          for (int q = 1; q < FW; q++) t = add4(t, red[((q * NS + s) * FRC + r) * WAVE + lane]);
-          if (b[s]) t = add4(t, load4w(b[s]));
-          v[s] = t;
-        }
-        float4 o = v[0];
-        if (MODE == MODE_UP)
-          o = make_float4(swiglu(v[0].x, v[1].x), swiglu(v[0].y, v[1].y), swiglu(v[0].z, v[1].z),
-                          swiglu(v[0].w, v[1].w));
-        store4(out + (int64_t)perm[p0 + r0 + r] * p.N + c0, o);
+        for (int j = 0; j < 4; j++) d.a[t][j] = xr[t][k + j < p.K ? k + j : 0];
       }
     }
-    __syncthreads();  // xs and red are rewritten by the next chunk
+  };
+  floatx4 tot[RT][4];
+#pragma unroll
+  for (int t = 0; t < RT; t++)
+#pragma unroll
+    for (int c = 0; c < 4; c++) tot[t][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](int s, const Step &d) {
+    floatx4 a[RT], b[4];
+#pragma unroll
+    for (int t = 0; t < RT; t++) a[t] = wide(d.a[t]);
+#pragma unroll
+    for (int j = 0; j < 4; j++) b[j] = wide(d.b[j]);
+    if (KF != K_STEPS) {  // k past K count as zeros (their weights read as zeros)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int t = 0; t < RT; t++) a[t][j] = s * FSTEP + 4 * kq + j < p.K ? a[t][j] : 0.f;
+    }
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+      for (int t = 0; t < RT; t++) {
+        floatx4 v = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          v = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][j], b[j][c], v, 0, 0, 0);
+        tot[t][c] = tot[t][c] + v;
+      }
+  };
+  Step ring[FPD];
+#pragma unroll
+  for (int j = 0; j < FPD - 1; j++) load(s0 + j, ring[j]);
+  for (int s = s0; s < s1; s += FPD) {
+#pragma unroll
+    for (int j = 0; j < FPD; j++) {
+      load(s + j + FPD - 1, ring[(j + FPD - 1) % FPD]);
+      __builtin_amdgcn_sched_barrier(0);  // the loads go out before this step's products
+      if (j == 0 || s + j < s1) compute(s + j, ring[j]);
+    }
+  }
+  // tot[t][c][q]: row 16t + 4kq + q, column col + c.
+#pragma unroll
+  for (int t = 0; t < RT; t++)
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      red[wave][4 * t + q][lane] = floatx4{tot[t][0][q], tot[t][1][q], tot[t][2][q], tot[t][3][q]};
+  __syncthreads();
+  if (!col_ok) return;
+  OT *out = (OT *)p.out + call * p.out_cs;
+  for (int i = wave; i < 4 * RT; i += FWAVES) {
+    const int r = 16 * (i >> 2) + 4 * kq + (i & 3);
+    if (r >= rows) continue;
+    floatx4 v[NS];
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      v[s] = red[s * KW][i][lane];
+#pragma unroll
+      for (int g = 1; g < KW; g++) v[s] = v[s] + red[s * KW + g][i][lane];
+      const WT *b = (const WT *)(s ? p.b1 : p.b0);
+      if (b) v[s] = v[s] + wide(load4(b + call * (s ? p.b1_cs : p.b0_cs) + (int64_t)e * p.N + col));
+    }
+    floatx4 u = v[0];
+    if constexpr (MODE == MODE_UP) {
+#pragma unroll
+      for (int c = 0; c < 4; c++) u[c] = swiglu(v[0][c], v[1][c]);
+    }
+    store4(out + (int64_t)perm[r] * p.N + col, u);
   }
 }
 
@@ -175,8 +251,48 @@ int launch_idx_route(const float *idx, int M, float *route, hipStream_t s) {
   return 0;
 }
 
-size_t float_expert_lds(int K, int mode, int fw, int frc) {
-  return (size_t)frc * K * 4 + (size_t)fw * (mode == MODE_UP ? 2 : 1) * frc * WAVE * 16;
+// Rows of the row stage of former versions: a K past it stays refused.
+static bool float_k_ok(int K, int mode, bool small) {
+  const int fw = small ? 8 : 4, frc = small ? 2 : 4;
+  return (size_t)frc * K * 4 + (size_t)fw * (mode == MODE_UP ? 2 : 1) * frc * WAVE * 16 <= 64 * 1024;
+}
+
+// Rows per tile, from the rows an expert has on average (block of 640 × 640, E
+// 128, top-4, µs, 16- and 32-row tiles: f32 150 tokens 143, 147, 300 tokens
+// 156, 155, 500 tokens 192, 171; f16, whose tiles cost half the bytes, 500
+// tokens 134, 142).
+int float_tile_rows(int A, int max_active, moe_dtype w_dt) {
+  return A / max_active <= (w_dt == MOE_F16 ? 16 : 6) ? 16 : 32;
+}
+
+template <int MODE, typename AT, typename WT, typename OT>
+static void launch_float_tile(const FloatArgs &p, int rows, int max_active, int calls, hipStream_t s) {
+  const int gx = (p.N + FCOLS - 1) / FCOLS;
+  const int64_t tiles = (int64_t)(p.db.A - max_active) / rows + max_active;
+  const dim3 grid((unsigned)((tiles * gx + 7) / 8 * 8), calls), block(FWAVES * WAVE);
+  const bool vx = p.K % 4 == 0 && (uintptr_t)p.a % (4 * sizeof(AT)) == 0 && p.a_cs % 4 == 0;
+  const int kf = !vx ? K_ANY : p.K % FSTEP ? K_QUADS : K_STEPS;
+  // 16-row tiles that fill the CUs twice: no step ahead, the registers for
+  // more wavefronts instead (77 tokens f32 133 → 123 µs a block, 150 tokens 143
+  // → 129, f16 99 → 95); fewer blocks: one ahead (4 tokens 44 → 41).
+  const bool full = tiles * gx >= 512;
+#define FLT_KF(RT_, KF_)                                                                            \
+  do {                                                                                              \
+    if (RT_ == 1 && full)                                                                           \
+      hipLaunchKernelGGL((k_float_tile<MODE, AT, WT, OT, RT_, KF_, 1>), grid, block, 0, s, p, gx);  \
+    else                                                                                            \
+      hipLaunchKernelGGL((k_float_tile<MODE, AT, WT, OT, RT_, KF_, 2>), grid, block, 0, s, p, gx);  \
+  } while (0)
+#define FLT_RT(RT_)                                \
+  do {                                             \
+    if (kf == K_STEPS) FLT_KF(RT_, K_STEPS);       \
+    else if (kf == K_QUADS) FLT_KF(RT_, K_QUADS);  \
+    else FLT_KF(RT_, K_ANY);                       \
+  } while (0)
+  if (rows == 16) FLT_RT(1);
+  else FLT_RT(2);
+#undef FLT_RT
+#undef FLT_KF
 }
 
 int launch_float_expert(const FloatArgs &p, int mode, moe_dtype a_dt, moe_dtype w_dt,
@@ -186,20 +302,16 @@ int launch_float_expert(const FloatArgs &p, int mode, moe_dtype a_dt, moe_dtype 
   MOE_NONNULL(p.out);
   MOE_NONNULL(p.db.perm);
   MOE_NONNULL(p.db.active);
+  MOE_NONNULL(p.db.meta);
   if (mode == MODE_UP) MOE_NONNULL(p.w1);
-  // Experts with at most ~2 rows on average (decode): 8 wavefronts × 2 rows.
-  const bool small = (long)p.db.A <= 2l * max_active;
-  const int fw = small ? 8 : 4, frc = small ? 2 : 4;
-  const size_t lds = float_expert_lds(p.K, mode, fw, frc);
-  if (lds > 64 * 1024)
+  if (!float_k_ok(p.K, mode, (long)p.db.A <= 2l * max_active))
     return moe_fail(MOE_INVALID_ARGUMENT, "float expert: K " + std::to_string(p.K) +
                                               " is too long for the 64 KB row stage");
-  dim3 grid((p.N + FCOLS - 1) / FCOLS, max_active, calls), block(fw * WAVE);
-#define FLT(M_, A_, W_, O_)                                                                   \
-  do {                                                                                        \
-    if (small) hipLaunchKernelGGL((k_float_expert<M_, A_, W_, O_, 8, 2, 8>), grid, block, lds, s, p); \
-    else hipLaunchKernelGGL((k_float_expert<M_, A_, W_, O_, 4, 4, 4>), grid, block, lds, s, p);       \
-  } while (0)
+  const int rows = float_tile_rows(p.db.A, max_active, w_dt);
+  if (((int64_t)p.db.A + max_active) * ((p.N + FCOLS - 1) / FCOLS) > 0x7ffffff0)
+    return moe_fail(MOE_INVALID_ARGUMENT, "float expert: too many rows");
+  if (p.N > (1 << 24)) return moe_fail(MOE_INVALID_ARGUMENT, "float expert: more than 2^24 columns");
+#define FLT(M_, A_, W_, O_) launch_float_tile<M_, A_, W_, O_>(p, rows, max_active, calls, s)
   const bool af = a_dt == MOE_F16, wf = w_dt == MOE_F16, of = o_dt == MOE_F16;
   if (mode == MODE_UP) {
     // act is f32 (the layer keeps its intermediates in f32)

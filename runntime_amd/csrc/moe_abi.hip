@@ -824,7 +824,8 @@ extern "C" int moe_matmul_gather(moe_ctx *ctx, const void *a, moe_dtype dtype, c
   {
     ProfScope ps(ctx, PG_DISPATCH);
     if ((rc = launch_idx_route(expert_idx, M, L.route, s))) return rc;
-    if ((rc = launch_dispatch(L.route, 0, M, E, 1, 1, TILE_M, L.db, s))) return rc;
+    if ((rc = launch_dispatch(L.route, 0, M, E, 1, 1, float_tile_rows(M, M < E ? M : E, dtype),
+                              L.db, s))) return rc;
   }
   {
     ProfScope ps(ctx, PG_DOWN);
@@ -864,6 +865,8 @@ extern "C" int moe_block_float(moe_ctx *ctx, const void *x, moe_dtype dtype, con
           "moe_block_float: NULL tensor");
   REQUIRE(eps > 0.f, "moe_block_float: eps must be positive, got " + std::to_string(eps));
   const int A = T * k;
+  const int max_active = A < E ? A : E;
+  const int tile_m = float_tile_rows(A, max_active, dtype);
   const size_t esize = dtype == MOE_F16 ? 2 : 4;
   LayerWs L;
   if ((rc = plan_ws(ctx, 1, T, k, E, route_out ? 0 : (size_t)T * 2 * k,
@@ -881,13 +884,12 @@ extern "C" int moe_block_float(moe_ctx *ctx, const void *x, moe_dtype dtype, con
   {
     ProfScope ps(ctx, PG_ROUTER);
     RouterArgs ra{L.xn, dtype, 0, w_router, 0, b_router, 0, route, 0, L.partial, T, d, E, k, 1};
-    if ((rc = launch_router_topk(ra, &L.db, TILE_M, &dispatched, s))) return rc;
+    if ((rc = launch_router_topk(ra, &L.db, tile_m, &dispatched, s))) return rc;
   }
   if (!dispatched) {
     ProfScope ps(ctx, PG_DISPATCH);
-    if ((rc = launch_dispatch(route, 0, T, E, k, 1, TILE_M, L.db, s))) return rc;
+    if ((rc = launch_dispatch(route, 0, T, E, k, 1, tile_m, L.db, s))) return rc;
   }
-  const int max_active = A < E ? A : E;
   {
     ProfScope ps(ctx, PG_UP);
     FloatArgs fa{};

@@ -332,6 +332,8 @@ struct FloatArgs {
   int64_t out_cs;
   DispatchBufs db;
 };
+// The dispatch counts M-tiles of float_tile_rows(...) rows.
+int float_tile_rows(int A, int max_active, moe_dtype w_dt);
 int launch_float_expert(const FloatArgs &p, int mode, moe_dtype a_dt, moe_dtype w_dt,
                         moe_dtype o_dt, int max_active, int calls, hipStream_t s);
 // route [M, 2] = {idx[i], 1} for a one-slot gather.

@@ -1,0 +1,136 @@
+"""The f32 matrix-core kernels at the edges of their tiles, against f64:
+k_linear (row tiles of 16 and 32, column tiles of 16, 32 and 64, K in whole
+steps, quads or any), k_sdpa_mfma (row tiles, key steps, key parts) and
+k_float_tile (row tiles of 16 and 32, K forms)."""
+import numpy as np
+import pytest
+import torch
+
+import runntime_amd as rt
+from oracle import ref
+from runntime_amd.linear import Linear
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+
+
+# (T, K, N): 16 x 16 tiles up to 32 x 64 ones, the last of each partly empty;
+# K of one step, past a step by 4 and by 1, fewer steps than wavefronts.
+@pytest.mark.parametrize("T,K,N", [(1, 16, 1), (17, 20, 33), (16, 640, 64), (65, 640, 1152),
+                                   (31, 132, 70), (321, 896, 644), (1000, 24, 260), (700, 647, 66),
+                                   (160, 33, 1600)])
+def test_linear_tiles(T, K, N):
+    print(f"linear T={T} K={K} N={N}", flush=True)
+    rng = np.random.default_rng(T + N)
+    x, w = rng.standard_normal((T, K)).astype(np.float32), rng.standard_normal((K, N)).astype(np.float32)
+    b, a = rng.standard_normal(N).astype(np.float32), rng.standard_normal((T, N)).astype(np.float32)
+    got = Linear(K, N, _dev(w), _dev(b)).forward(_dev(x), _dev(a)).cpu().numpy()
+    xd, wd = x.astype(np.float64), w.astype(np.float64)
+    want = xd @ wd + b + a
+    mag = np.abs(xd) @ np.abs(wd) + np.abs(b) + np.abs(a)
+    # chains of at most 32 products, then K / 32 sums, 8 parts, bias and addend
+    np.testing.assert_array_less(np.abs(got - want), (32 + K / 32 + 12) * 2.0 ** -24 * mag + 1e-30)
+
+
+def test_linear_keeps_infinities_in_their_rows():
+    print("linear infinities", flush=True)
+    x = np.ones((40, 20), np.float32)
+    x[7, 3], x[39, 19] = np.inf, np.nan
+    w = np.ones((20, 33), np.float32)
+    w[0, 5] = np.inf
+    got = Linear(20, 33, _dev(w)).forward(_dev(x)).cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        want = x.astype(np.float64) @ w.astype(np.float64)
+    np.testing.assert_array_equal(got, want.astype(np.float32))
+
+
+ATTN = [  # q_len, kv_len, q_heads, kv_heads, head_dim, left, right, offset, extra
+    (1, 1, 2, 2, 64, -1, -1, 0, ""), (1, 300, 14, 2, 64, -1, -1, 299, ""),
+    (15, 15, 14, 2, 64, 128, 128, 0, "sinks"), (17, 33, 3, 1, 128, 5, 0, 16, "sinks"),
+    (33, 64, 8, 1, 64, 0, 0, 31, ""), (64, 64, 4, 2, 128, 40, 40, 0, "segments"),
+    (97, 97, 9, 1, 64, 31, 7, 0, "segments sinks"), (50, 200, 2, 1, 64, -1, -1, 0, "bias"),
+    (300, 300, 16, 2, 64, 128, 128, 0, "sinks"), (700, 700, 18, 2, 64, 30, 30, 0, "sinks")]
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+@pytest.mark.parametrize("c", ATTN, ids=[f"q{c[0]}kv{c[1]}h{c[2]}-{c[3]}d{c[4]}" for c in ATTN])
+def test_sdpa_tiles(dtype, c):
+    qn, kn, qh, kh, hd, left, right, off, extra = c
+    print(f"sdpa tiles {dtype} {c}", flush=True)
+    rng = np.random.default_rng(qn + kn)
+    npd = np.float16 if dtype == "f16" else np.float32
+    q = (rng.standard_normal((qn, qh * hd)) * hd ** -0.25).astype(npd)
+    k = (rng.standard_normal((kn, kh * hd)) * hd ** -0.25).astype(npd)
+    v = rng.standard_normal((kn, kh * hd)).astype(npd)
+    inf = float("inf")
+    opts = {"qHeads": qh, "kvHeads": kh, "headDim": hd, "windowLeft": inf if left < 0 else left,
+            "windowRight": inf if right < 0 else right, "qPosOffset": off}
+    sinks = rng.standard_normal(qh).astype(np.float32) if "sinks" in extra else None
+    segs = None
+    if "segments" in extra:  # rows 10 to 19 see nothing
+        cut = np.array([0, kn // 3, kn // 2, kn])
+        seg = np.searchsorted(cut, np.arange(qn), side="right") - 1
+        segs = np.stack([cut[seg], cut[seg + 1]], 1).astype(np.float32)
+        segs[10:20] = (4, 4)
+    score = np.zeros((qh, qn, kn))
+    out = np.zeros((qn, qh * hd))
+    pos = off + np.arange(qn)[:, None]
+    key = np.arange(kn)[None, :]
+    seen = np.ones((qn, kn), bool)
+    if left >= 0:
+        seen &= key >= pos - left
+    if right >= 0:
+        seen &= key <= pos + right
+    if segs is not None:
+        seen &= (key >= segs[:, :1]) & (key < segs[:, 1:])
+    kb = {"start": 3, "end": kn // 2, "value": -1.5} if "bias" in extra else None
+    for h in range(qh):
+        g = h // (qh // kh)
+        s = q[:, h * hd:(h + 1) * hd].astype(np.float64) @ k[:, g * hd:(g + 1) * hd].astype(np.float64).T
+        if kb:
+            s[:, kb["start"]:kb["end"]] += kb["value"]
+        e = np.where(seen, np.exp(s - s.max(1, keepdims=True)), 0.0)
+        den = e.sum(1, keepdims=True)
+        if sinks is not None:
+            den = den + np.exp(float(sinks[h]) * np.log(2.0) - s.max(1, keepdims=True))
+        out[:, h * hd:(h + 1) * hd] = np.divide(e, den, out=np.zeros_like(e), where=den > 0) \
+            @ v[:, g * hd:(g + 1) * hd].astype(np.float64)
+    if sinks is not None:
+        opts["sinks"] = _dev(sinks)
+    if segs is not None:
+        opts["segments"] = _dev(segs)
+    if kb:
+        opts["keyBias"] = kb
+    got = rt.sdpa(_dev(q), _dev(k), _dev(v), opts).float().cpu().numpy()
+    # f32 sums of head_dim and of the probabilities; f16 outputs round to 11 bits
+    np.testing.assert_allclose(got, out, atol=(2e-5 if dtype == "f32" else 1e-3 * np.abs(v).max()),
+                               rtol=(1e-4 if dtype == "f32" else 1e-3))
+
+
+# Rows per expert from one to a second 32-row tile; K whole steps, past one by
+# 4, and odd; N a partial column block; many blocks (no step ahead) and few.
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+@pytest.mark.parametrize("M,K,N,E", [(1, 16, 4, 1), (33, 36, 68, 2), (200, 640, 132, 40),
+                                     (130, 19, 64, 3), (90, 48, 260, 90), (700, 260, 72, 16)])
+def test_float_tiles(dtype, M, K, N, E):
+    print(f"float tiles {dtype} M={M} K={K} N={N} E={E}", flush=True)
+    rng = np.random.default_rng(M + K)
+    npd = np.float16 if dtype == "f16" else np.float32
+    a = rng.standard_normal((M, K)).astype(npd)
+    w = rng.standard_normal((E * K, N)).astype(npd)
+    b = rng.standard_normal((E, N)).astype(npd)
+    idx = rng.integers(0, E, M).astype(np.float32)
+    idx[::9] = -1.0
+    got = rt.matmulGather(_dev(a), _dev(w), _dev(idx), {"bias": _dev(b)}).float().cpu().numpy()
+    want, mag = np.zeros((M, N)), np.zeros((M, N))
+    for e in range(E):
+        r, we = idx == e, w[e * K:(e + 1) * K].astype(np.float64)
+        want[r] = a[r].astype(np.float64) @ we + b[e]
+        mag[r] = np.abs(a[r].astype(np.float64)) @ np.abs(we) + np.abs(b[e].astype(np.float64))
+    eps = (16 + K / 16 + 10) * 2.0 ** -24
+    bound = eps * mag + (2.0 ** -11 * np.abs(want) + 1e-7 if dtype == "f16" else 0.0) + 1e-30
+    np.testing.assert_array_less(np.abs(got - want), bound)
