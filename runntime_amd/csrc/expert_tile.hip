@@ -113,8 +113,20 @@ struct APlanes {
 template <typename AT, int RT>
 constexpr int tile_kc() { return sizeof(AT) == 4 && RT > 1 ? 64 : 128; }
 
+// Wavefronts per SIMD the registers are kept to. 64-row tiles of int8 with
+// plain scales: three (the block of d 640, E 128, top-4, I 640 at 1500
+// tokens: 101.2 us, 102.9 at two). 16-row tiles of three planes: three, since
+// they spill at four (int4 layer of 64 tokens 62.8 us instead of 65, of 300
+// tokens 70 instead of 73).
+template <typename AT, int BITS, bool GROUPED, int RT>
+constexpr int tile_waves() {
+  if (RT == 4) return BITS == 8 && !GROUPED ? 3 : 2;
+  return RT == 2 || APlanes<AT, BITS>::BF ? 3 : 4;
+}
+
 template <int MODE, typename AT, int BITS, bool GROUPED, int RT>
-__global__ __launch_bounds__(64 * TW) __attribute__((amdgpu_waves_per_eu(RT == 4 ? 2 : RT == 2 ? 3 : 4)))
+__global__ __launch_bounds__(64 * TW) __attribute__((
+    amdgpu_waves_per_eu(tile_waves<AT, BITS, GROUPED, RT>())))
 void k_expert_tile(TileArgs p) {
   typedef APlanes<AT, BITS> AP;
   constexpr int ROWS = 16 * RT;
@@ -129,6 +141,10 @@ void k_expert_tile(TileArgs p) {
   constexpr int PER = ROWS * KC / 8 / (64 * TW);  // 8-value pieces per thread
   static_assert(PER >= 1, "at least one load per thread");
   constexpr int PPR = KC / 8;               // such pieces per row
+  // 16-row tiles: the sums of a piece start from zero and join the total, so
+  // chains of additions are short (2.5e-7 of a layer's result instead of
+  // 5.2e-7 at K 2048); larger tiles have no registers for it.
+  constexpr bool FOLD = !GROUPED && RT == 1;
   extern __shared__ __align__(16) unsigned char smem[];
   uint16_t *abuf = (uint16_t *)smem;
   __shared__ int s_row[ROWS];  // rows of the dispatch's assignments
@@ -316,11 +332,23 @@ void k_expert_tile(TileArgs p) {
     }
   };
 
-  floatx4 tot[RT][4];
+  floatx4 tot[RT][4], acc[FOLD ? RT : 1][4];
 #pragma unroll
   for (int t = 0; t < RT; t++)
 #pragma unroll
-    for (int i = 0; i < 4; i++) tot[t][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < 4; i++) {
+      tot[t][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+      if (FOLD) acc[FOLD ? t : 0][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+  auto fold = [&]() {
+    if constexpr (FOLD) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        tot[0][i] += acc[0][i];
+        acc[0][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+  };
 
   auto mfma = [&](u32x4 a, u32x4 b, floatx4 c) -> floatx4 {
     if constexpr (AP::BF)
@@ -369,7 +397,10 @@ void k_expert_tile(TileArgs p) {
             tot[t][i] += v * d.s[h][i];
           } else {
 #pragma unroll
-            for (int q = AP::N - 1; q >= 0; q--) tot[t][i] = mfma(a[q][t], b, tot[t][i]);
+            for (int q = AP::N - 1; q >= 0; q--) {
+              floatx4 &c = FOLD ? acc[FOLD ? t : 0][i] : tot[t][i];
+              c = mfma(a[q][t], b, c);
+            }
           }
         }
       }
@@ -389,6 +420,7 @@ void k_expert_tile(TileArgs p) {
       issue(s + j + TPD - 1, ring[(j + TPD - 1) % TPD]);
       if (j == 0 || s + j < lsteps) compute(ring[j], abuf + cur * BUF, (j % CS) * LK);
       if (j % CS == CS - 1) {
+        fold();
         cur ^= 1;
         store_a((s + j + 1) * LK, abuf + cur * BUF);
         __syncthreads();
