@@ -10,7 +10,8 @@ Both kinds run on moe_linear (linear.hip): the weight is kept as f32 [in,
 out], a quantized one dequantized once at load (int · its group's scale,
 one f32 product per weight). The projections of this model are small (a
 few MB per block), and the texts are tens of rows, so the kernel spreads
-the work over columns and K slices rather than streaming int8.
+the work over tiles of rows and columns on the f32 matrix cores rather than
+streaming int8.
 """
 from dataclasses import dataclass
 from typing import Optional
