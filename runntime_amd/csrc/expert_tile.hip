@@ -31,9 +31,9 @@
 //
 // Bound by the weight stream while an expert has up to ~32 rows, by the
 // int8 → f16 conversions and MFMAs above. Measured (2048 × 1408, E 64, 300
-// tokens, top-8, f16 x): up 397 → 75-85 µs (369 MB, 4.4-4.9 TB/s), down
-// 208 → 52-60 µs against the skinny kernel, which takes 16 rows at a time
-// and streams (and converts) the weights once for each.
+// tokens, top-8, f16 x): layer 611 → 174 µs against the skinny kernel (up 397,
+// down 208), which takes 16 rows at a time and streams (and converts) the
+// weights once for each.
 // Ring of 4 load steps: 8 is no faster with plain scales and spills with
 // group scales (56 tokens int4 g 32: 76 → 130 µs a layer).
 #include "gemm_dev.h"
@@ -113,14 +113,14 @@ struct APlanes {
 template <typename AT, int RT>
 constexpr int tile_kc() { return sizeof(AT) == 4 && RT > 1 ? 64 : 128; }
 
-// Wavefronts per SIMD the registers are kept to. 64-row tiles of int8 with
-// plain scales: three (the block of d 640, E 128, top-4, I 640 at 1500
-// tokens: 101.2 us, 102.9 at two). 16-row tiles of three planes: three, since
-// they spill at four (int4 layer of 64 tokens 62.8 us instead of 65, of 300
-// tokens 70 instead of 73).
+// Wavefronts per SIMD the registers are kept to: what fits with at most a few
+// registers spilled. 64-row tiles of f32 rows under int8: three (two more
+// spilled values, but the block of d 640, E 128, top-4, I 640 at 1500 tokens
+// was 1.5% faster at three than at two). 16-row tiles of three planes: three,
+// since they spill at four (int4 layer of 64 tokens 62.8 us instead of 65).
 template <typename AT, int BITS, bool GROUPED, int RT>
 constexpr int tile_waves() {
-  if (RT == 4) return BITS == 8 && !GROUPED ? 3 : 2;
+  if (RT == 4) return BITS == 8 && !GROUPED && sizeof(AT) == 4 ? 3 : 2;
   return RT == 2 || APlanes<AT, BITS>::BF ? 3 : 4;
 }
 
@@ -141,10 +141,16 @@ void k_expert_tile(TileArgs p) {
   constexpr int PER = ROWS * KC / 8 / (64 * TW);  // 8-value pieces per thread
   static_assert(PER >= 1, "at least one load per thread");
   constexpr int PPR = KC / 8;               // such pieces per row
-  // 16-row tiles: the sums of a piece start from zero and join the total, so
-  // chains of additions are short (2.5e-7 of a layer's result instead of
-  // 5.2e-7 at K 2048); larger tiles have no registers for it.
-  constexpr bool FOLD = !GROUPED && RT == 1;
+  // No chain of additions runs over all of K: it would be longer, and its
+  // error larger, than that of the K-split streams this kernel stands in for
+  // (1536 x 1000, E 32, top-4, 500 tokens on few experts: 3.8e-7 of the
+  // result there, 4.3e-7 in one chain, 2.2e-7 so). FOLD: the sums of a piece
+  // start from zero and join the total. Larger tiles of several planes have
+  // no registers for that: every MFMA step's planes start from zero and join
+  // the total. It costs 64-row tiles some time (2048 x 1408, E 64, top-8, 300
+  // tokens of f16: layer 150 -> 174 us for 5.2e-7 -> 3.1e-7; d 640 at 1500
+  // tokens of f32: block 100 -> 112 us for 4.4e-7 -> 3.1e-7), 16-row tiles none.
+  constexpr bool FOLD = !GROUPED && (RT == 1 || (AP::N == 1 && BITS == 8));
   extern __shared__ __align__(16) unsigned char smem[];
   uint16_t *abuf = (uint16_t *)smem;
   __shared__ int s_row[ROWS];  // rows of the dispatch's assignments
@@ -343,10 +349,12 @@ void k_expert_tile(TileArgs p) {
   auto fold = [&]() {
     if constexpr (FOLD) {
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        tot[0][i] += acc[0][i];
-        acc[0][i] = floatx4{0.f, 0.f, 0.f, 0.f};
-      }
+      for (int t = 0; t < RT; t++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          tot[t][i] += acc[FOLD ? t : 0][i];
+          acc[FOLD ? t : 0][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
     }
   };
 
@@ -396,11 +404,13 @@ void k_expert_tile(TileArgs p) {
             for (int q = AP::N - 1; q >= 0; q--) v = mfma(a[q][t], b, v);
             tot[t][i] += v * d.s[h][i];
           } else {
+            floatx4 one = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int q = AP::N - 1; q >= 0; q--) {
-              floatx4 &c = FOLD ? acc[FOLD ? t : 0][i] : tot[t][i];
+              floatx4 &c = FOLD ? acc[FOLD ? t : 0][i] : one;
               c = mfma(a[q][t], b, c);
             }
+            if (!FOLD) tot[t][i] += one;
           }
         }
       }
@@ -520,7 +530,7 @@ bool expert_tile_eligible(const ExpertArgs &ea) {
 //     the skinny kernel, which splits K over wavefronts (one token: 33 there,
 //     36 here; 2048 × 1408 two tokens 57, 60), from three rows an expert or
 //     1000 wavefronts on it is this one (640 × 640 32 tokens 60 → 54;
-//     2048 × 1408 f16 64 tokens 237 → 151, 300 tokens 615 → 158).
+//     2048 × 1408 f16 64 tokens 232 → 121, 300 tokens 611 → 174).
 //   Row tile: as the rows an expert has on average, with room for their
 //     spread (2048 × 1408, 12 rows each: 150 with 16-row tiles, 127 with 32;
 //     24: 206, 153, 150 with 64; 48: 331, 243, 180), halved while the launch
