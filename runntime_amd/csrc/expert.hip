@@ -360,9 +360,9 @@ __global__ __launch_bounds__(64 * NWS * KS) __attribute__((amdgpu_waves_per_eu(N
     sc[j] = second ? p.s1 + call * p.s1_cs : p.s0 + call * p.s0_cs;
     const float *b = second ? (p.b1 ? p.b1 + call * p.b1_cs : nullptr)
                             : (p.b0 ? p.b0 + call * p.b0_cs : nullptr);
-    const uint32_t slab = (uint32_t)p.K * (uint32_t)p.N * (uint32_t)p.bits / 8u;
-    wr[j] = __builtin_amdgcn_make_buffer_rsrc((void *)((const char *)w + (int64_t)e * slab), 0,
-                                              (int)slab, BUF_DWORD3);
+    const int64_t slab = quantw_bytes(p.K, p.N, 8);  // < 2^31 (skinny_takes)
+    wr[j] = __builtin_amdgcn_make_buffer_rsrc((void *)((const char *)w + e * slab), 0, (int)slab,
+                                              BUF_DWORD3);
 #pragma unroll
     for (int h2 = 0; h2 < 2; h2++) {
       const int u = (useg[j] & ~15) + 8 * h2 + (lane & 7);
@@ -816,9 +816,16 @@ __global__ void k_zero(float *__restrict__ p, size_t n) {
   for (; i < n; i += stride) p[i] = 0.f;
 }
 
+// k_expert_skinny's weights: int8, scale groups in whole MFMA steps, 32-bit
+// buffer offsets.
+bool skinny_takes(const ExpertArgs &ea) {
+  return ea.bits == 8 && (ea.g == ea.K || ea.g % 32 == 0) &&
+         quantw_bytes(ea.K, ea.N, 8) < (1ll << 31);
+}
+
 template <int MODE>
 int launch_mode(const ExpertArgs &ea, const ExpertKArgs &p, hipStream_t s) {
-  const bool mfma = ea.bits == 8 && (ea.g == ea.K || ea.g % 32 == 0);
+  const bool mfma = skinny_takes(ea);
   const int max_active = ea.E < ea.A ? ea.E : ea.A;
   if (mfma) {
     ExpertKArgs q = p;
@@ -926,8 +933,7 @@ bool expert_uses_gemm(const ExpertArgs &ea) {
 }
 
 bool expert_stages_norm(const ExpertArgs &ea) {
-  return ea.mode == MODE_UP && !ea.tile_rows && !expert_uses_gemm(ea) && ea.bits == 8 &&
-         (ea.g == ea.K || ea.g % 32 == 0);
+  return ea.mode == MODE_UP && !ea.tile_rows && !expert_uses_gemm(ea) && skinny_takes(ea);
 }
 
 bool expert_fuses_route(const ExpertArgs &up, int J) {

@@ -204,9 +204,9 @@ void k_expert_tile(TileArgs p) {
   const float *sc = (arr ? p.s1 + call * p.s1_cs : p.s0 + call * p.s0_cs) + (int64_t)e * kg * p.N;
   const float *bi = arr ? (p.b1 ? p.b1 + call * p.b1_cs : nullptr)
                         : (p.b0 ? p.b0 + call * p.b0_cs : nullptr);
-  const uint32_t slab = (uint32_t)p.K * (uint32_t)p.N * BITS / 8u;
+  const int64_t slab = quantw_bytes(p.K, p.N, BITS);  // < 2^31 (expert_tile_eligible)
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
-      (void *)((const char *)w + (int64_t)e * slab), 0, (int)slab, BUF_DWORD3);
+      (void *)((const char *)w + e * slab), 0, (int)slab, BUF_DWORD3);
   const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(
       (void *)sc, 0, (int)((uint32_t)kg * (uint32_t)p.N * 4u), BUF_DWORD3);
   // Loaded units and 16-byte chunks (a chunk: one int8 tile, 4 k, or two int4
@@ -517,7 +517,7 @@ bool expert_tile_eligible(const ExpertArgs &ea) {
                    : ea.bits == 4 || ea.a_dtype == MOE_F16 ? ea.K % 8 == 0 : ea.K % 4 == 0;
   return kok && (uintptr_t)ea.a % 16 == 0 && ea.a_cs * (ea.a_dtype == MOE_F16 ? 2 : 4) % 16 == 0 &&
          (ea.mode == MODE_UP || ea.a_dtype == MOE_F32) &&
-         (int64_t)ea.K * ea.N * ea.bits / 8 < (1ll << 31) &&
+         quantw_bytes(ea.K, ea.N, ea.bits) < (1ll << 31) &&
          (int64_t)(ea.K / ea.g) * ea.N * 4 < (1ll << 31);
 }
 

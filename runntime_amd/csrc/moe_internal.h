@@ -174,6 +174,15 @@ int launch_dispatch(const float *route, int64_t route_cs, int T, int E, int k, i
 
 enum ExpertMode { MODE_UP = 0, MODE_DOWN = 1 };
 
+// Bytes of one expert's quantW words, in 64 bits: K·N·bits passes 2^32 from
+// 512 MiB on.
+__host__ __device__ constexpr int64_t quantw_bytes(int K, int N, int bits) {
+  return (int64_t)K * N / 8 * bits;
+}
+static_assert(quantw_bytes(32768, 32768, 4) == 1ll << 29, "2^30 int4 weights");
+static_assert(quantw_bytes(4096, 131072, 8) == 1ll << 29, "2^29 int8 weights");
+static_assert(quantw_bytes(32768, 65536, 8) == 1ll << 31, "past 32-bit buffer offsets");
+
 struct ExpertArgs {
   int mode;                 // ExpertMode
   const void *a;            // x [T, K] (up) or act [T·k, K] (down)

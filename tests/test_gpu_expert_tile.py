@@ -122,6 +122,40 @@ def test_int4_f32_range():
     assert np.isnan(out[4]).all()
 
 
+def _unit_columns(words, e, u, K, N, bits):
+    """Expert e's columns 4u .. 4u + 3 as f64 [K, 4], from quantW words."""
+    n = K // 4 * bits // 2
+    w = words[(e * (N // 4) + u) * n:][:n].view(torch.int8).to(torch.int32)
+    v = w if bits == 8 else torch.stack([(w << 28) >> 28, w >> 4], -1)
+    return v.reshape(K // 4, 4, 4).transpose(1, 2).reshape(K, 4).double()
+
+
+# Experts of 2^29 bytes of weights, where K·N·bits is 2^32: one row an expert
+# and several (int8: k_expert_skinny, then k_expert_tile).
+@pytest.mark.parametrize("bits,K,N,T", [(4, 32768, 32768, 4), (8, 4096, 131072, 2),
+                                        (8, 4096, 131072, 6)])
+def test_experts_of_half_a_gib(bits, K, N, T):
+    print(f"large experts int{bits} {K} x {N} T={T}", flush=True)
+    E = 2
+    g = torch.Generator(device=DEV).manual_seed(bits + T)
+    words = torch.randint(-(1 << 31), 1 << 31, (E * K * N * bits // 32,), generator=g, device=DEV,
+                          dtype=torch.int64).to(torch.int32)
+    sc = torch.rand((E, N), generator=g, device=DEV) + 0.5
+    a = torch.randn((T, K), generator=g, device=DEV)
+    route = torch.ones((T, 2), device=DEV)
+    route[:, 0] = torch.arange(T, device=DEV) % E
+    w = rt.QuantExpertWeight(rt.QuantW(words, (E * K, N)), sc, None)
+    out = rt.moeDown(a, route, w, None, {"bits": bits, "groupSize": K})
+    for u in (0, 1, N // 8 + 3, N // 4 - 1):
+        for e in range(E):
+            q = _unit_columns(words, e, u, K, N, bits)
+            s = sc[e, 4 * u:4 * u + 4].double()
+            rows = a[e::E].double()
+            got, want = out[e::E, 4 * u:4 * u + 4].double(), rows @ q * s
+            bound = ((K / 32 + 8) * 2.0 ** -23 + 2.0 ** -21) * (rows.abs() @ q.abs()) * s
+            assert torch.all((got - want).abs() <= bound), (u, e)
+
+
 # Layers on each side of the rules: few rows per expert on wide weights, row
 # tiles of 16, 32 and 64, K not a multiple of 32 (I = 1000), and the grouped
 # GEMM's forms from 80 (f16 x: int8 limbs, an odd number of step pairs; f16
