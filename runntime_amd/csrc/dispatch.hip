@@ -116,6 +116,14 @@ constexpr int ONE_WAVES = 16;
 constexpr int ONE_MAX_A = ONE_WAVES * WAVE * 8;
 constexpr int ONE_MAX_E = 512;  // (16 + 2)·E counts in LDS: 37 KB
 
+// Orders the wavefront's LDS accesses before and after it (no instruction:
+// the LDS serves a wavefront in order).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <int NC>
 __global__ __launch_bounds__(ONE_WAVES *WAVE) void k_dispatch_one(const float *__restrict__ route,
                                                                   int64_t route_cs, int A, int k,
@@ -175,12 +183,14 @@ __global__ __launch_bounds__(ONE_WAVES *WAVE) void k_dispatch_one(const float *_
       const uint64_t ones = __ballot(e >= 0 && ((e >> bit) & 1));
       same &= ((e >> bit) & 1) ? ones : ~ones;
     }
+    const int rank = __popcll(same & ((1ull << lane) - 1ull));
+    const int32_t base = e >= 0 ? mine[e] : 0;
+    wave_sync();  // every lane has read before the first one of an expert adds
     if (e >= 0) {
-      const int rank = __popcll(same & ((1ull << lane) - 1ull));
-      const int32_t base = mine[e];  // every lane reads before the first one adds
       perm[off[e] + base + rank] = a0 + i * WAVE;
       if (rank == 0) mine[e] = base + __popcll(same);
     }
+    wave_sync();  // and the next chunk reads what this one wrote
   }
   for (int i = off[E] + threadIdx.x; i < A; i += ONE_WAVES * WAVE) perm[i] = -1;
 }

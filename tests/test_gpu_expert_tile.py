@@ -206,6 +206,21 @@ def test_dispatch_one_block(T, k, E):
     np.testing.assert_array_equal(perm.cpu().numpy(), want_perm)
 
 
+@pytest.mark.parametrize("T,hot", [(8192, 64), (8192, 1), (5000, 3), (1100, 2)])
+def test_dispatch_experts_across_chunks(T, hot):
+    """One block, up to eight chunks a wavefront, and an expert with rows in all
+    of them: a chunk's places follow on those the chunk before it counted."""
+    print(f"dispatch chunks T={T} hot={hot}", flush=True)
+    E = 128
+    route = np.ones((T, 2), np.float32)
+    t = np.arange(T)
+    route[:, 0] = np.where(t % 64 < hot, 7, t * 31 % E)
+    perm, off = rt.dispatch(torch.from_numpy(route).to(DEV), E)
+    want_perm, _, want_off = ref.dispatch(route, E)
+    np.testing.assert_array_equal(off.cpu().numpy(), want_off)
+    np.testing.assert_array_equal(perm.cpu().numpy(), want_perm)
+
+
 @pytest.mark.parametrize("E,k", [(7, 3), (64, 8), (130, 4), (513, 16)])
 def test_topk_special_logits(E, k):
     """Infinities, NaN, both zeros (equal, the lower id first), values at and
