@@ -456,79 +456,133 @@ __global__ __launch_bounds__(512) void k_sdpa_mfma(AttnArgs a, int hw, int kspli
   for (int b = 0; b < NB; b++)
 #pragma unroll
     for (int c = 0; c < 4; c++) acc[b][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto scores = [&](const KTile &kt, floatx4 (&sc)[NT]) {
+#pragma unroll
+    for (int n = 0; n < NT; n++) {
+      // two chains: halves the dependent MFMA latency
+      floatx4 s0 = floatx4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+      for (int s = 0; s < NS; s++) {
+        floatx4 k4;
+        if constexpr (ROPE)
+          k4 = rope4(kt.k[n][s], kt.c[n][s], kt.s[n][s]);
+        else
+          k4 = floatx4{kt.k[n][s].x, kt.k[n][s].y, kt.k[n][s].z, kt.k[n][s].w};
+        s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[0], q[s][0], s0, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[1], q[s][1], s1, 0, 0, 0);
+        s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[2], q[s][2], s0, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[3], q[s][3], s1, 0, 0, 0);
+      }
+      sc[n] = s0 + s1;
+    }
+  };
+  // Scores of step st to probabilities under the running max; returns the
+  // factor for what was summed before.
+  auto softmax = [&](int st, floatx4 (&sc)[NT]) -> float {
+    const int key0 = blo + st * KC + 4 * g;
+    float top = -INFINITY;
+#pragma unroll
+    for (int n = 0; n < NT; n++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int key = key0 + 16 * n + j;
+        float x = sc[n][j];
+        if (a.has_kb && key >= a.kb_start && key < a.kb_end) x += a.kb_value;
+        x = key >= lo && key <= hi ? x : -INFINITY;
+        sc[n][j] = x;
+        top = fmaxf(top, x);
+      }
+    top = fmaxf(top, __shfl_xor(top, 16));
+    top = fmaxf(top, __shfl_xor(top, 32));
+    const float mn = fmaxf(mx, top);
+    const float base = mn == -INFINITY ? 0.f : mn;  // nothing seen yet
+    const float scale = mx == -INFINITY ? 0.f : expf(mx - base);
+    float add = 0.f;
+#pragma unroll
+    for (int n = 0; n < NT; n++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int key = key0 + 16 * n + j;
+        const float p = key >= lo && key <= hi ? expf(sc[n][j] - base) : 0.f;
+        sc[n][j] = p;
+        add += p;
+      }
+    add += __shfl_xor(add, 16);
+    add += __shfl_xor(add, 32);
+    sum = sum * scale + add;
+    mx = mn;
+    return scale;
+  };
+  // P·V of head columns (b, c); keys outside klo .. khi count as V = 0.
+  auto pv = [&](int b, int c, const floatx4 (&sc)[NT], bool masked, int key0, int klo, int khi) {
+    floatx4 o = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int n = 0; n < NT; n++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const float4 &vv = v[n][j][b];
+        float ve = c == 0 ? vv.x : c == 1 ? vv.y : c == 2 ? vv.z : vv.w;
+        if (masked) ve = key0 + 16 * n + j >= klo && key0 + 16 * n + j <= khi ? ve : 0.f;
+        o = __builtin_amdgcn_mfma_f32_16x16x4f32(ve, sc[n][j], o, 0, 0, 0);
+      }
+    return o;
+  };
   if (c_first < c_last) {  // then blo ≤ bhi: every address is a key's
     KTile kt;
     load_k(c_first, kt);
     load_v(c_first);
     for (int st = c_first; st < c_last; st++) {
       floatx4 sc[NT];
-#pragma unroll
-      for (int n = 0; n < NT; n++) {
-        // two chains: halves the dependent MFMA latency
-        floatx4 s0 = floatx4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
-#pragma unroll
-        for (int s = 0; s < NS; s++) {
-          floatx4 k4;
-          if constexpr (ROPE)
-            k4 = rope4(kt.k[n][s], kt.c[n][s], kt.s[n][s]);
-          else
-            k4 = floatx4{kt.k[n][s].x, kt.k[n][s].y, kt.k[n][s].z, kt.k[n][s].w};
-          s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[0], q[s][0], s0, 0, 0, 0);
-          s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[1], q[s][1], s1, 0, 0, 0);
-          s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[2], q[s][2], s0, 0, 0, 0);
-          s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[3], q[s][3], s1, 0, 0, 0);
-        }
-        sc[n] = s0 + s1;
-      }
+      scores(kt, sc);
       load_k(min(st + 1, c_last - 1), kt);  // lands under the softmax and P·V
-      const int key0 = blo + st * KC + 4 * g;
-      float top = -INFINITY;
-#pragma unroll
-      for (int n = 0; n < NT; n++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const int key = key0 + 16 * n + j;
-          float x = sc[n][j];
-          if (a.has_kb && key >= a.kb_start && key < a.kb_end) x += a.kb_value;
-          x = key >= lo && key <= hi ? x : -INFINITY;
-          sc[n][j] = x;
-          top = fmaxf(top, x);
-        }
-      top = fmaxf(top, __shfl_xor(top, 16));
-      top = fmaxf(top, __shfl_xor(top, 32));
-      const float mn = fmaxf(mx, top);
-      const float base = mn == -INFINITY ? 0.f : mn;  // nothing seen yet
-      const float scale = mx == -INFINITY ? 0.f : expf(mx - base);
-      float add = 0.f;
-#pragma unroll
-      for (int n = 0; n < NT; n++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const int key = key0 + 16 * n + j;
-          const float p = key >= lo && key <= hi ? expf(sc[n][j] - base) : 0.f;
-          sc[n][j] = p;
-          add += p;
-        }
-      add += __shfl_xor(add, 16);
-      add += __shfl_xor(add, 32);
-      sum = sum * scale + add;
-      mx = mn;
+      const float scale = softmax(st, sc);
 #pragma unroll
       for (int b = 0; b < NB; b++)
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-          floatx4 o = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int n = 0; n < NT; n++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-              const float4 &vv = v[n][j][b];
-              const float ve = c == 0 ? vv.x : c == 1 ? vv.y : c == 2 ? vv.z : vv.w;
-              o = __builtin_amdgcn_mfma_f32_16x16x4f32(ve, sc[n][j], o, 0, 0, 0);
-            }
-          acc[b][c] = acc[b][c] * scale + o;
-        }
+        for (int c = 0; c < 4; c++)
+          acc[b][c] = acc[b][c] * scale + pv(b, c, sc, false, 0, 0, 0);
       load_v(min(st + 1, c_last - 1));
+    }
+  }
+  // The V operand is shared by the tile's rows, and 0 times an infinity or a
+  // NaN of a key that a row does not see is NaN. Such a NaN stays in acc, so
+  // the loop above needs no test; where one came out, the keys are walked
+  // again, P·V for one row after the other with the V it does not see zeroed.
+  bool nan = false;
+#pragma unroll
+  for (int b = 0; b < NB; b++)
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) nan |= acc[b][c][i] != acc[b][c][i];
+  if (__any(nan)) {
+    mx = -INFINITY;
+    sum = 0.f;
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+      for (int c = 0; c < 4; c++) acc[b][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int st = c_first; st < c_last; st++) {
+      floatx4 sc[NT];
+      {
+        KTile kt;
+        load_k(st, kt);
+        scores(kt, sc);
+      }
+      const float scale = softmax(st, sc);
+      load_v(st);
+#pragma unroll 1
+      for (int r = 0; r < 16; r++) {
+        const int rlo = __builtin_amdgcn_readlane(lo, r), rhi = __builtin_amdgcn_readlane(hi, r);
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+          for (int c = 0; c < 4; c++) {
+            const floatx4 o = pv(b, c, sc, true, blo + st * KC + 4 * g, rlo, rhi);
+            if (m == r) acc[b][c] = acc[b][c] * scale + o;
+          }
+      }
     }
   }
   // acc[b][c][i]: row `row`, head column 64b + 16g + 4i + c.

@@ -111,6 +111,41 @@ def test_sdpa_tiles(dtype, c):
                                rtol=(1e-4 if dtype == "f32" else 1e-3))
 
 
+# An infinity or a NaN in V reaches the rows that see its key, and no other row
+# of its 16-row tile: one step of keys, several, keys split over wavefronts,
+# several heads a block; the last key, which pads a tile's last step.
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+@pytest.mark.parametrize("n,qh,kh,hd,left,right", [(70, 4, 2, 64, 9, 4), (70, 3, 1, 128, 40, 3),
+                                                   (300, 14, 2, 64, 60, 60), (500, 72, 8, 64, 5, 0)])
+def test_sdpa_keeps_infinities_from_rows_that_do_not_see_them(dtype, n, qh, kh, hd, left, right):
+    print(f"sdpa infinities {dtype} {n} {qh}/{kh} {hd} {left} {right}", flush=True)
+    rng = np.random.default_rng(n + hd)
+    npd = np.float16 if dtype == "f16" else np.float32
+    q = (rng.standard_normal((n, qh * hd)) * hd ** -0.25).astype(npd)
+    k = (rng.standard_normal((n, kh * hd)) * hd ** -0.25).astype(npd)
+    v = rng.standard_normal((n, kh * hd)).astype(npd)
+    v[20], v[33, 3::5], v[n - 1, ::2] = np.inf, np.nan, -np.inf
+    cut = np.array([0, 21, n // 2, n])
+    seg = np.searchsorted(cut, np.arange(n), side="right") - 1
+    segs = np.stack([cut[seg], cut[seg + 1]], 1).astype(np.float32)
+    segs[10] = (4, 4)
+    want = np.zeros((n, qh * hd))
+    for r in range(n):
+        lo, hi = int(max(r - left, segs[r, 0])), int(min(r + right + 1, segs[r, 1]))
+        for h in range(qh if hi > lo else 0):
+            c, g = slice(h * hd, (h + 1) * hd), h // (qh // kh)
+            cg = slice(g * hd, (g + 1) * hd)
+            s = k[lo:hi, cg].astype(np.float64) @ q[r, c].astype(np.float64)
+            e = np.exp(s - s.max())
+            with np.errstate(invalid="ignore"):
+                want[r, c] = (e / e.sum()) @ v[lo:hi, cg].astype(np.float64)
+    got = rt.sdpa(_dev(q), _dev(k), _dev(v),
+                  {"qHeads": qh, "kvHeads": kh, "headDim": hd, "windowLeft": left, "windowRight": right,
+                   "segments": _dev(segs)}).float().cpu().numpy()
+    np.testing.assert_allclose(got, want, atol=2e-5 if dtype == "f32" else 4e-3,
+                               rtol=1e-4 if dtype == "f32" else 1e-3)
+
+
 # Rows per expert from one to a second 32-row tile; K whole steps, past one by
 # 4, and odd; N a partial column block; many blocks (no step ahead) and few.
 @pytest.mark.parametrize("dtype", ["f32", "f16"])
