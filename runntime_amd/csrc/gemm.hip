@@ -385,10 +385,9 @@ void k_expert_gemm(GemmArgs p) {
     uint32_t hl[CT];
 #pragma unroll
     for (int c = 0; c < CT; c += 2) {
-      const _Float16 h0 = (_Float16)v[c], h1 = (_Float16)v[c + 1];
-      hl[c] = __builtin_bit_cast(uint32_t, half2v{h0, h1});
-      hl[c + 1] = __builtin_bit_cast(
-          uint32_t, half2v{(_Float16)(v[c] - (float)h0), (_Float16)(v[c + 1] - (float)h1)});
+      const u32x2 parts = f16_parts(v[c], v[c + 1]);
+      hl[c] = parts[0];
+      hl[c + 1] = parts[1];
     }
     if constexpr (CT == 4)
       __builtin_amdgcn_raw_buffer_store_b128(u32x4{hl[0], hl[1], hl[2], hl[3]}, orc, off, 0, 0);

@@ -138,6 +138,18 @@ __device__ __forceinline__ void dma4(i32x4 rsrc, uint32_t voff, int soff, uint32
                :: "v"(voff), "s"(rsrc), "s"(soff), "s"(lds_addr) : "memory");
 }
 
+// Two f32 values as f16 hi and lo parts: {hi(a), hi(b)} and {lo(a), lo(b)}.
+// The empty asm makes each value the rounded f32 one. Without it the compiler
+// merges the multiply that made it into each conversion on its own
+// (v_fma_mixlo_f16): the hi that is stored and the hi that lo completes could
+// then differ by a last f16 bit, and hi + lo be off by it.
+__device__ __forceinline__ u32x2 f16_parts(float a, float b) {
+  asm("" : "+v"(a), "+v"(b));
+  const _Float16 ha = (_Float16)a, hb = (_Float16)b;
+  return u32x2{__builtin_bit_cast(uint32_t, half2v{ha, hb}),
+               __builtin_bit_cast(uint32_t, half2v{(_Float16)(a - (float)ha), (_Float16)(b - (float)hb)})};
+}
+
 // s_waitcnt with vmcnt = n (< 64) and no wait on the other counters.
 #define WAIT_VMCNT(n) \
   __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))

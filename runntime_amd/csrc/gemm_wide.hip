@@ -331,10 +331,7 @@ void k_gemm_up_direct(GemmArgs p) {
           u32x2 o;
           if constexpr (OMODE == 1) {
             // The f32 pair's 8 bytes as hi(n), hi(n + 1), lo(n), lo(n + 1).
-            const _Float16 h0 = (_Float16)v[0], h1 = (_Float16)v[1];
-            o[0] = __builtin_bit_cast(uint32_t, half2v{h0, h1});
-            o[1] = __builtin_bit_cast(
-                uint32_t, half2v{(_Float16)(v[0] - (float)h0), (_Float16)(v[1] - (float)h1)});
+            o = f16_parts(v[0], v[1]);
           } else {
             o[0] = __builtin_bit_cast(uint32_t, v[0]);
             o[1] = __builtin_bit_cast(uint32_t, v[1]);

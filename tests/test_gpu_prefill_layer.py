@@ -62,3 +62,21 @@ def test_prefill_layer_int8_limbs(cfg):
     if cfg.zipf:
         assert (counts == 0).any(), "the skewed shape should leave an expert without rows"
     assert_close(got, want, what=f"{cfg.name} output")
+
+
+@pytest.mark.parametrize("cfg", [MoeConfig("e_f32x", 512, 1024, 8, 2, 1024, "f32"),
+                                 MoeConfig("e_i1056", 512, 1024, 8, 2, 1056, "f16")],
+                         ids=lambda c: c.name)
+def test_prefill_act_pairs_keep_f32(cfg):
+    """act as f16 hi + lo pairs between the products (up with f32 x; up with f16
+    x on I = 1056) is f32's 22 bits: the layer is within 2^-20 of f64 (norm over
+    norm; each product's parts are good to 2^-22, its f32 sums to about 2^-21).
+    A pair whose hi is not the one its lo completes is off by 2^-11 of a value."""
+    print(f"prefill pairs {cfg}", flush=True)
+    inp = make_inputs(cfg, seed=21, keep_q=True, bias_rand=True)
+    inp.residual.zero_()
+    out = rt.moe_layer(inp.x, inp.router_w, inp.router_b, inp.glu, inp.lin, inp.down, inp.residual,
+                       cfg.k)
+    got = out.cpu().numpy().astype(np.float64)
+    _, want = _oracle(inp, cfg)
+    assert np.linalg.norm(got - want) <= 2.0 ** -20 * np.linalg.norm(want)
