@@ -227,6 +227,14 @@ MOE_API int moe_block(moe_ctx *ctx, const void *x, moe_dtype x_dtype, const void
 MOE_API int moe_rmsnorm(moe_ctx *ctx, const void *x, moe_dtype dtype, int rows, int cols,
                         const void *weight, int weight_len, float eps, int group,
                         const void *residual, float scale, void *out);
+/* Which kernel the expert products of these sizes run on: rows per tile of
+ * each, 128 for the grouped GEMM, 16, 32 or 64 for k_expert_tile, 0 for the
+ * decode kernels. op 0: moe_up (down_rows -1), 1: moe_down (K = I, N = d;
+ * up_rows -1), 2: moe_layer, or moe_layer_batched with `calls` calls. Host
+ * only, for 16-byte aligned tensors; no counterpart in the reference. */
+MOE_API int moe_expert_tiles(int op, int calls, moe_dtype x_dtype, int T, int d, int I, int E,
+                             int k, int bits, int group_size_up, int group_size_down,
+                             int *up_rows, int *down_rows);
 /* matmulGather(a, w, expertIdx, {bias}) (src/core/graph/ops/matmul.ts:180-210):
  * out[i] = a[i]·W[e_i] + bias[e_i], W = rows [e·K, (e+1)·K) of the float
  * weight w [E·K, N] (row-major), e_i = expert_idx[i] (f32 [M], exact

@@ -28,7 +28,7 @@ EXPORTED = (
     "moe_block", "moe_rmsnorm", "moe_matmul_gather", "moe_block_float", "moe_rope",
     "moe_sdpa", "moe_linear", "moe_viterbi_decode", "moe_attention", "moe_ctx_pin_workspace",
     "moe_check_expert_weight", "moe_buffer_alloc", "moe_buffer_free", "moe_buffer_write",
-    "moe_buffer_read", "moe_layer_noalloc",
+    "moe_buffer_read", "moe_layer_noalloc", "moe_expert_tiles",
 )
 PROF_GROUPS = ("topk", "router", "dispatch", "up", "down", "combine", "norm")
 
@@ -109,6 +109,7 @@ def load() -> ctypes.CDLL:
             "moe_matmul_gather": ([P, P, I, P, P, P, I, I, I, I, P], I),
             "moe_block_float": ([P, P, I, P, ctypes.c_float, P, P, P, P, P, P, P, P, I, I, I, I, I,
                                  P, P], I),
+            "moe_expert_tiles": ([I] * 11 + [ctypes.POINTER(I)] * 2, I),
             "moe_rope": ([P, P, I, I, I, I, I, I, P, P, P], I),
             "moe_linear": ([P, P, P, P, P, I, I, I, P], I),
             "moe_viterbi_decode": ([P, P, P, P, I, I, P], I),

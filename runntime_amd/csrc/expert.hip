@@ -23,7 +23,7 @@
 //
 // Where the rows per expert or the weights' form ask for it, k_expert_tile
 // (expert_tile.hip) or the grouped GEMM (gemm*.hip) runs instead: the rules
-// are at expert_tile_rows and gemm_min_rows.
+// are at expert_tile_rows and gemm_pays.
 //
 // k_expert_simple — VALU fallback for what is left (scale groups that are
 // not a multiple of 32, int4 with a K or an alignment k_expert_tile does not
@@ -907,29 +907,13 @@ int launch_mode(const ExpertArgs &ea, const ExpertKArgs &p, hipStream_t s) {
 
 }  // namespace
 
-// Where the grouped GEMM's 128-row tiles and once-converted weights beat
-// k_expert_tile's 64-row ones (µs, GEMM against tile, rows per expert):
-//   layers with f16 x: 2048 × 1408 64 rows 229, 224; 80 rows 243, 277; 640
-//     rows 1065, 1369. Short K or N never: its ring and 256-column tiles
-//     do not pay off (640 × 640 96 rows 154, 139; 640 rows 590, 569).
-//   layers with f32 x: from 64 rows, as callers have had it. The tile kernel
-//     is faster there too (640 × 640 64 rows 156, 126), but its f32 act and
-//     this path's f16-pair act differ by 5e-6 of the result, more than the
-//     2e-6 that results may move by.
-//   moe_up alone, f16 x: 640 × 640 96 rows 70, 78; 256 rows 123, 131.
-//   moe_up (f32 x) and moe_down alone: 2048 × 1408 128 rows 367, 269 and 193,
-//     161; 512 rows 893, 881 and 483, 491; 640 × 640 always the tile kernel.
-int gemm_min_rows(bool x_f16, int K, int N, bool layer) {
-  const bool wide = K >= 1024 && N >= 1024;
-  if (x_f16) return wide || !layer ? 80 : INT32_MAX;
-  return layer ? 64 : wide ? 512 : INT32_MAX;
-}
-
+// Arguments that both take: the grouped GEMM from 64 rows an expert if
+// gemm_pays says so, else k_expert_tile. What k_expert_tile does not take:
+// from 64 rows.
 bool expert_uses_gemm(const ExpertArgs &ea) {
   const int max_active = ea.E < ea.A ? ea.E : ea.A;
-  // Arguments k_expert_tile does not take: from 64 rows an expert.
-  const int64_t rows = expert_tile_eligible(ea) ? ea.gemm_rows : 64;
-  return ea.calls == 1 && ea.A >= rows * max_active && gemm_eligible(ea);
+  return ea.calls == 1 && ea.A >= (int64_t)64 * max_active && gemm_eligible(ea) &&
+         (!expert_tile_eligible(ea) || ea.gemm_pays);
 }
 
 bool expert_stages_norm(const ExpertArgs &ea) {

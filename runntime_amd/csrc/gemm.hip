@@ -673,14 +673,53 @@ int gemm_down_parts(const ExpertArgs &ea) {
   if (ea.mode != MODE_DOWN || !gemm_eligible(ea)) return 1;
   const int ksteps = ea.K / BK;
   if (ksteps % 2 || ksteps / 2 < 3 * gemm_stages(ea)) return 1;
-  const long cus = gemm_cus();
-  if (cus <= 0) return 1;
+  const long cus = gemm_cus() > 0 ? gemm_cus() : 256;  // no device: the rule is still asked
   // Rounds of whole tiles over the CUs against rounds of half tiles (each
   // half as long), from the upper bound of the tile count.
   const long tiles = gemm_mtiles(ea) * ((ea.N + 511) / 512);
   const long whole = (tiles + cus - 1) / cus;
   const long halves = (2 * tiles + cus - 1) / cus;
   return halves < 2 * whole ? 2 : 1;
+}
+
+// Where the grouped GEMM beats k_expert_tile (from 64 rows an expert). Its
+// persistent blocks go over the CUs in whole passes of 128-row tiles (256
+// columns in up, 512 in down), where k_expert_tile's 64-row blocks spread
+// finely. So the line is the fill of its passes: rows × columns over what they
+// could hold. An expert counts as one row tile while hardly any has more than
+// 128 rows, then with half a tile of padding.
+//
+// Measured on 850 shapes of 64 to 2048 rows an expert (8 to 128 experts, K and
+// N 512 to 5632, random routers), GEMM time over tile time below the line and
+// from it, median (least, most):
+//   layer, f16 x   1.18 (0.88, 2.01)   0.87 (0.62, 1.08)
+//   layer, f32 x   1.51 (1.24, 2.35)   1.02 (0.74, 1.38)
+//   up, f16 x      1.13 (0.82, 1.37)   0.80 (0.61, 1.06)
+//   up, f32 x      1.21 (1.01, 2.51)   0.95 (0.80, 1.06)
+//   down           1.18 (0.97, 2.18)   0.93 (0.75, 1.03)
+// For instance 2048 × 1408, E 64, layer with f16 x, µs: 64 rows 229, 239; 128
+// rows 341, 369; 512 rows 884, 1199; 640 × 640: 128 rows 120, 99; 2048 × 5632, E
+// 32: 64 rows 361, 473. Short K has a higher line: a tile's fixed part weighs
+// more. Layers with f32 x keep the GEMM as far as it is faster anywhere.
+// A layer whose up the GEMM does not take stays whole on k_expert_tile (512 ×
+// 1024, f16 x, E 32, 64 to 512 rows: 94 to 169, 57 to 168).
+bool gemm_pays(const ExpertArgs &ea, bool layer) {
+  if (!gemm_eligible(ea)) return false;
+  const bool up = ea.mode == MODE_UP;
+  const int max_active = ea.E < ea.A ? ea.E : ea.A;
+  const int cus = gemm_cus() > 0 ? gemm_cus() : 256;
+  const int cols = up ? 256 : 512;
+  const double avg = (double)ea.A / max_active;
+  const double parts = up ? 1 : gemm_down_parts(ea);
+  const double mtiles = max_active * (avg < 105 ? 1.0 : avg / BM + 0.5);
+  const int64_t passes =
+      (int64_t)((mtiles * ((ea.N + cols - 1) / cols) * parts + cus - 1) / cus);
+  const double fill =
+      (double)ea.A / BM * ea.N / cols * parts / ((double)cus * (passes > 1 ? passes : 1));
+  const bool one = passes <= 1;
+  if (!up) return one ? fill >= 0.5 : fill >= 0.65 && (parts == 1 || passes <= 2);
+  if (ea.a_dtype != MOE_F16) return fill >= (layer ? 0.3 : one ? 0.5 : 0.66);
+  return fill >= (ea.K >= 1024 ? 0.22 : ea.N >= 1024 ? 0.3 : one || !layer ? 0.38 : 0.55);
 }
 
 int launch_expert_gemm(const ExpertArgs &ea, const DispatchBufs &db, hipStream_t s) {

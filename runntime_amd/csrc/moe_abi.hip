@@ -478,6 +478,65 @@ extern "C" int moe_pack_quantw(moe_ctx *ctx, const int8_t *ints, int E, int k, i
   return after_launch("packQuantW");
 }
 
+// The kernel of a product alone, and of the two of a layer. The dispatch
+// counts M-tiles (returned) in the row tile that both products use, else in
+// the grouped GEMM's, which k_expert_tile then splits.
+static void plan_product(ExpertArgs &ea) {
+  ea.gemm_pays = gemm_pays(ea, false);
+  ea.tile_rows = expert_tile_rows(ea);
+  ea.tile_m = ea.tile_rows ? ea.tile_rows : TILE_M;
+}
+static int plan_layer(ExpertArgs &up, ExpertArgs &dn) {
+  up.gemm_pays = dn.gemm_pays = gemm_pays(up, true);
+  up.tile_rows = expert_tile_rows(up);
+  dn.tile_rows = expert_tile_rows(dn);
+  if (up.tile_rows && dn.tile_rows) dn.tile_rows = up.tile_rows;
+  up.tile_m = dn.tile_m =
+      up.tile_rows && up.tile_rows == dn.tile_rows ? up.tile_rows : TILE_M;
+  return up.tile_m;
+}
+
+extern "C" int moe_expert_tiles(int op, int calls, moe_dtype x_dtype, int T, int d, int I, int E,
+                                int k, int bits, int group_size_up, int group_size_down,
+                                int *up_rows, int *down_rows) {
+  REQUIRE(op >= 0 && op <= 2 && calls >= 1 && T >= 1 && d >= 1 && I >= 1 && E >= 1 && k >= 1 &&
+              group_size_up >= 1 && group_size_down >= 1 && up_rows && down_rows,
+          "expert tiles: bad argument");
+  ExpertArgs up{}, dn{};
+  up.mode = MODE_UP;
+  up.a_dtype = x_dtype;
+  up.a_row_div = k;
+  dn.mode = MODE_DOWN;
+  dn.a_dtype = MOE_F32;
+  dn.a_row_div = 1;
+  up.K = dn.N = d;
+  up.N = dn.K = I;
+  up.g = group_size_up;
+  dn.g = group_size_down;
+  for (ExpertArgs *ea : {&up, &dn}) {
+    ea->k = k;
+    ea->E = E;
+    ea->bits = bits;
+    ea->A = T * k;
+    ea->calls = calls;
+  }
+  if (calls > 1) up.a_cs = (int64_t)T * d;
+  dn.a_cs = (int64_t)T * k * I;
+  if (op == 2) {
+    plan_layer(up, dn);
+  } else {
+    dn.a_cs = 0;
+    plan_product(up);
+    plan_product(dn);
+  }
+  auto rows = [](const ExpertArgs &ea) {
+    return ea.tile_rows ? ea.tile_rows : expert_uses_gemm(ea) ? TILE_M : 0;
+  };
+  *up_rows = op == 1 ? -1 : rows(up);
+  *down_rows = op == 0 ? -1 : rows(dn);
+  return MOE_OK;
+}
+
 extern "C" int moe_up(moe_ctx *ctx, const void *x, moe_dtype x_dtype, const float *route,
                       const moe_expert_weight *glu, const moe_expert_weight *lin, int T, int K,
                       int N, int E, int k, int bits, int group_size, float *act) {
@@ -494,7 +553,6 @@ extern "C" int moe_up(moe_ctx *ctx, const void *x, moe_dtype x_dtype, const floa
   ea.mode = MODE_UP;
   ea.a = x;
   ea.a_dtype = x_dtype;
-  ea.gemm_rows = gemm_min_rows(x_dtype == MOE_F16, K, N, false);
   ea.a_row_div = k;
   ea.route = route;
   ea.k = k;
@@ -508,8 +566,7 @@ extern "C" int moe_up(moe_ctx *ctx, const void *x, moe_dtype x_dtype, const floa
   ea.out = act;
   ea.A = T * k;
   ea.calls = 1;
-  ea.tile_rows = expert_tile_rows(ea);
-  ea.tile_m = ea.tile_rows ? ea.tile_rows : TILE_M;
+  plan_product(ea);
   {
     ProfScope ps(ctx, PG_DISPATCH);
     if ((rc = launch_dispatch(route, 0, T, E, k, 1, ea.tile_m, L.db, ctx->stream))) return rc;
@@ -548,10 +605,8 @@ extern "C" int moe_down(moe_ctx *ctx, const float *act, const float *route,
   ea.g = group_size;
   ea.A = T * k;
   ea.calls = 1;
-  ea.gemm_rows = gemm_min_rows(false, K, N, false);
+  plan_product(ea);
   ea.parts = expert_uses_gemm(ea) ? gemm_down_parts(ea) : 1;
-  ea.tile_rows = expert_tile_rows(ea);
-  ea.tile_m = ea.tile_rows ? ea.tile_rows : TILE_M;
   LayerWs L;
   if ((rc = plan_ws(ctx, 1, T, k, E, 0, 0, 0, (size_t)ea.parts * T * k * N, L))) return rc;
   ea.out = L.y;
@@ -614,7 +669,6 @@ static int layer_impl(const char *op, moe_ctx *ctx, int calls, const moe_call_st
   up.mode = MODE_UP;
   up.a = x;
   up.a_dtype = x_dtype;
-  up.gemm_rows = dn.gemm_rows = gemm_min_rows(x_dtype == MOE_F16, d, I, true);
   up.a_cs = st->x;
   up.a_row_div = k;
   up.k = k;
@@ -650,13 +704,7 @@ static int layer_impl(const char *op, moe_ctx *ctx, int calls, const moe_call_st
   dn.g = group_size_down;
   dn.A = A;
   dn.calls = calls;
-  up.tile_rows = expert_tile_rows(up);
-  dn.tile_rows = expert_tile_rows(dn);
-  if (up.tile_rows && dn.tile_rows) dn.tile_rows = up.tile_rows;
-  // The dispatch counts M-tiles in the row tile both products use, else in
-  // the grouped GEMM's (k_expert_tile then splits them).
-  const int tile_m = up.tile_rows && up.tile_rows == dn.tile_rows ? up.tile_rows : TILE_M;
-  up.tile_m = dn.tile_m = tile_m;
+  const int tile_m = plan_layer(up, dn);
   // Both products on the grouped GEMM: act stays in dispatch order, so down
   // streams each tile's rows contiguously instead of gathering them; down
   // may split K in two partial products, which the combine adds.

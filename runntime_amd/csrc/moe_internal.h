@@ -235,9 +235,9 @@ struct ExpertArgs {
   // 0: they do not), and the M-tile rows the dispatch counted with.
   int tile_rows;
   int tile_m;
-  // Rows per expert (average) from which the grouped GEMM takes over from
-  // k_expert_tile (gemm_min_rows, one value for both products of a layer).
-  int gemm_rows;
+  // The grouped GEMM is faster than k_expert_tile here (gemm_pays, one value
+  // for both products of a layer).
+  bool gemm_pays;
 };
 
 int launch_expert(const ExpertArgs &ea, const DispatchBufs &db, hipStream_t s);
@@ -264,9 +264,8 @@ bool gemm_wide_eligible(const ExpertArgs &ea);
 // these arguments, else 0.
 int expert_tile_rows(const ExpertArgs &ea);
 bool expert_tile_eligible(const ExpertArgs &ea);
-// ExpertArgs::gemm_rows for products with K and N columns; `layer` for the
-// two products of a layer, whose act has a form of its own on the GEMM.
-int gemm_min_rows(bool x_f16, int K, int N, bool layer);
+// ExpertArgs::gemm_pays of a product, or of a layer from its up product.
+bool gemm_pays(const ExpertArgs &ea, bool layer);
 int launch_expert_tile(const ExpertArgs &ea, const DispatchBufs &db, hipStream_t s);
 int64_t gemm_i8_act_bytes(int A, int E, int K);
 int launch_expert_gemm(const ExpertArgs &ea, const DispatchBufs &db, hipStream_t s);

@@ -69,3 +69,17 @@ def swiglu_np(g, l):
     g = np.minimum(g, 7.0)
     l = np.clip(l, -7.0, 7.0)
     return g / (1.0 + np.exp(-1.702 * g)) * (l + 1.0)
+
+
+def expert_tiles(op, T, d, I, E, k, x_dtype, bits=8, group_up=None, group_down=None, calls=1):
+    """(up, down) rows per tile of the kernels that moe_up ("up"; down is None),
+    moe_down ("down"; K = I, N = d) or moe_layer ("layer") takes: 128 the
+    grouped GEMM, 16, 32 or 64 k_expert_tile, 0 the decode kernels."""
+    import ctypes
+
+    from runntime_amd import _lib
+    up, down = ctypes.c_int(), ctypes.c_int()
+    _lib.check(_lib.load().moe_expert_tiles(
+        ("up", "down", "layer").index(op), calls, 1 if x_dtype == "f16" else 0, T, d, I, E, k, bits,
+        group_up or d, group_down or I, ctypes.byref(up), ctypes.byref(down)))
+    return (None if op == "down" else up.value, None if op == "up" else down.value)
