@@ -69,7 +69,10 @@ __device__ __forceinline__ typename Cols<CT>::type load_cols(__amdgpu_buffer_rsr
 
 // CT > 1 needs N a multiple of CT and the pointers other than x aligned to CT
 // floats.
-enum KForm { K_STEPS = 0, K_QUADS = 1, K_ANY = 2 };  // K % 16 == 0, % 4 == 0 (x aligned), any
+// K % 16 == 0, % 4 == 0 (x aligned), any; any with rows of W so wide that 16 of
+// them pass the buffer offsets (64-bit addresses, CT = 1)
+enum KForm { K_STEPS = 0, K_QUADS = 1, K_ANY = 2, K_WIDE = 3 };
+constexpr int L_MAX_N = 1 << 24;
 template <int RT, int CT, int KW, int KF>
 __global__ __launch_bounds__(64 * KW) void k_linear(const float *__restrict__ x,
                                                     const float *__restrict__ w,
@@ -109,17 +112,26 @@ __global__ __launch_bounds__(64 * KW) void k_linear(const float *__restrict__ x,
     const int k = s * LSTEP + 4 * kq;
 #pragma unroll
     for (int t = 0; t < RT; t++) {
-      if constexpr (KF != K_ANY) {
+      if constexpr (KF == K_STEPS || KF == K_QUADS) {
         d.a[t] = *(const floatx4 *)(xr[t] + (KF == K_STEPS || k < K ? k : 0));
       } else {
 #pragma unroll
         for (int j = 0; j < 4; j++) d.a[t][j] = xr[t][k + j < K ? k + j : 0];
       }
     }
-    const int left = KF == K_STEPS ? LSTEP : min(LSTEP, K - s * LSTEP);
-    const __amdgpu_buffer_rsrc_t wr = rows_rsrc(w + (int64_t)s * LSTEP * N, left * N * 4);
+    if constexpr (KF == K_WIDE) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) d.b[j] = load_cols<CT>(wr, woff[j]);
+      for (int j = 0; j < 4; j++) {
+        const bool ok = k + j < K && col < N;
+        const float v = w[ok ? (int64_t)(k + j) * N + col : 0];
+        d.b[j][0] = ok ? v : 0.f;
+      }
+    } else {
+      const int left = KF == K_STEPS ? LSTEP : min(LSTEP, K - s * LSTEP);
+      const __amdgpu_buffer_rsrc_t wr = rows_rsrc(w + (int64_t)s * LSTEP * N, left * N * 4);
+#pragma unroll
+      for (int j = 0; j < 4; j++) d.b[j] = load_cols<CT>(wr, woff[j]);
+    }
   };
   floatx4 acc[RT][CT], tot[RT][CT];
 #pragma unroll
@@ -207,7 +219,6 @@ int launch_linear(const float *x, const float *w, const float *bias, const float
   MOE_NONNULL(y);
   if ((T + 15) / 16 > 65535)
     return moe_fail(MOE_INVALID_ARGUMENT, "linear: more than " + std::to_string(65535 * 16) + " rows");
-  if (N > (1 << 24)) return moe_fail(MOE_INVALID_ARGUMENT, "linear: more than 2^24 columns");
   auto aligned = [](const void *p, int bytes) { return (uintptr_t)p % bytes == 0; };
   const bool vx = K % 4 == 0 && aligned(x, 16);
   auto cols_ok = [&](int ct) {
@@ -222,11 +233,12 @@ int launch_linear(const float *x, const float *w, const float *bias, const float
   // block, µs, at 1500 rows 180, 238, 266; 300 rows 77, 85, 89; 150 rows 66,
   // 63, 65; the network at 110 rows 894, 837, 858; at 32 rows 715, 661, 639.
   int rt = 1, ct = 1;
-  if (vx && cols_ok(4) && blocks(2, 4) >= 100) rt = 2, ct = 4;
-  else if (vx && cols_ok(2) && blocks(1, 2) >= 130) ct = 2;
+  const bool wide = N > L_MAX_N;
+  if (!wide && vx && cols_ok(4) && blocks(2, 4) >= 100) rt = 2, ct = 4;
+  else if (!wide && vx && cols_ok(2) && blocks(1, 2) >= 130) ct = 2;
   const int64_t n = blocks(rt, ct);
   if (n > 0x7fffffff) return moe_fail(MOE_INVALID_ARGUMENT, "linear: output too large");
-  const int ncb = (N + 16 * ct - 1) / (16 * ct);
+  const int ncb = (int)(((int64_t)N + 16 * ct - 1) / (16 * ct));
 #define LIN_KF(RT_, CT_, KW_, KF_)                                                                \
   hipLaunchKernelGGL((k_linear<RT_, CT_, KW_, KF_>), dim3((unsigned)n), dim3(64 * KW_), 0, s, x, w, \
                      bias, addend, y, T, K, N, ncb)
@@ -235,7 +247,8 @@ int launch_linear(const float *x, const float *w, const float *bias, const float
     if (K % LSTEP == 0) LIN_KF(RT_, CT_, KW_, K_STEPS);      \
     else LIN_KF(RT_, CT_, KW_, K_QUADS);                     \
   } while (0)
-  if (rt == 2) LIN(2, 4, 4);
+  if (wide) LIN_KF(1, 1, 8, K_WIDE);
+  else if (rt == 2) LIN(2, 4, 4);
   else if (ct == 2) LIN(1, 2, 8);
   else if (vx) LIN(1, 1, 8);
   else LIN_KF(1, 1, 8, K_ANY);

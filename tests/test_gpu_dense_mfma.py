@@ -36,6 +36,28 @@ def test_linear_tiles(T, K, N):
     np.testing.assert_array_less(np.abs(got - want), (32 + K / 32 + 12) * 2.0 ** -24 * mag + 1e-30)
 
 
+# Rows of W so wide that 16 of them pass 32-bit offsets; K past a step, T past a
+# row tile, an infinity in W's first row (K past K reads must not meet it).
+@pytest.mark.parametrize("T,K,N", [(1, 3, (1 << 24) + 1), (17, 18, (1 << 24) + 35)])
+def test_linear_more_than_2p24_columns(T, K, N):
+    print(f"linear T={T} K={K} N={N}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(K)
+    x = torch.randn((T, K), generator=g, device=DEV)
+    w = torch.randn((K, N), generator=g, device=DEV)
+    w[0, 5] = float("inf")
+    b = torch.randn(N, generator=g, device=DEV)
+    a = torch.randn((T, N), generator=g, device=DEV)
+    got = Linear(K, N, w, b).forward(x, a)
+    for c in (slice(0, 40), slice(N // 2 - 9, N // 2 + 50), slice(N - 60, N)):
+        wc, bc, ac = w[:, c].double(), b[c].double(), a[:, c].double()
+        want = torch.stack([(x[:, k:k + 1].double() * wc[k]) for k in range(K)]).sum(0) + bc + ac
+        mag = (x.double().abs() @ wc.abs()) + bc.abs() + ac.abs()
+        fin = torch.isfinite(want)
+        assert torch.equal(got[:, c].double()[~fin], want[~fin])
+        err = (got[:, c].double() - want)[fin].abs()
+        assert torch.all(err <= (32 + 12) * 2.0 ** -24 * mag[fin] + 1e-30)
+
+
 def test_linear_keeps_infinities_in_their_rows():
     print("linear infinities", flush=True)
     x = np.ones((40, 20), np.float32)
