@@ -78,7 +78,10 @@ template <> struct Vec4<_Float16> { typedef half4 type; };
 // MODE_UP: act[a] = swiglu(x·glu[e] + bias_glu[e], x·lin[e] + bias_lin[e]).
 // MODE_DOWN (and the plain gather): out[a] = x·w[e] + bias[e].
 // AT: activation type, WT: weight and bias type, OT: output type.
-enum KForm { K_STEPS = 0, K_QUADS = 1, K_ANY = 2 };  // K % 16 == 0, % 4 == 0 (rows of a aligned), any
+// K % 16 == 0, % 4 == 0 (rows of a aligned), any; any with weight rows so wide
+// that 16 of them pass the buffer offsets (64-bit addresses)
+enum KForm { K_STEPS = 0, K_QUADS = 1, K_ANY = 2, K_WIDE = 3 };
+constexpr int F_MAX_N = 1 << 24;
 // FPD: steps loaded (the one multiplied and those ahead of it).
 template <int MODE, typename AT, typename WT, typename OT, int RT, int KF, int FPD>
 __global__ __launch_bounds__(FWAVES *WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_float_tile(FloatArgs p, int gx) {
@@ -150,14 +153,24 @@ __global__ __launch_bounds__(FWAVES *WAVE) __attribute__((amdgpu_waves_per_eu(4)
   auto load = [&](int s, Step &d) {
     s = min(s, steps - 1);
     const int k = s * FSTEP + 4 * kq;
-    const int left = KF == K_STEPS ? FSTEP : min(FSTEP, p.K - s * FSTEP);
-    const __amdgpu_buffer_rsrc_t wr =
-        rows_rsrc(w + (int64_t)s * FSTEP * p.N, left * p.N * (int)sizeof(WT));
+    if constexpr (KF == K_WIDE) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) stream4(d.b[j], wr, woff[j]);
+      for (int j = 0; j < 4; j++) {
+        const bool ok = k + j < p.K && col_ok;
+        const wv4 v = load4(w + (ok ? (int64_t)(k + j) * p.N + col : 0));
+#pragma unroll
+        for (int c = 0; c < 4; c++) d.b[j][c] = ok ? v[c] : (WT)0;
+      }
+    } else {
+      const int left = KF == K_STEPS ? FSTEP : min(FSTEP, p.K - s * FSTEP);
+      const __amdgpu_buffer_rsrc_t wr =
+          rows_rsrc(w + (int64_t)s * FSTEP * p.N, left * p.N * (int)sizeof(WT));
+#pragma unroll
+      for (int j = 0; j < 4; j++) stream4(d.b[j], wr, woff[j]);
+    }
 #pragma unroll
     for (int t = 0; t < RT; t++) {
-      if constexpr (KF != K_ANY) {
+      if constexpr (KF == K_STEPS || KF == K_QUADS) {
         d.a[t] = load4(xr[t] + (KF == K_STEPS || k < p.K ? k : 0));
       } else {
 #pragma unroll
@@ -267,7 +280,7 @@ int float_tile_rows(int A, int max_active, moe_dtype w_dt) {
 
 template <int MODE, typename AT, typename WT, typename OT>
 static void launch_float_tile(const FloatArgs &p, int rows, int max_active, int calls, hipStream_t s) {
-  const int gx = (p.N + FCOLS - 1) / FCOLS;
+  const int gx = (int)(((int64_t)p.N + FCOLS - 1) / FCOLS);
   const int64_t tiles = (int64_t)(p.db.A - max_active) / rows + max_active;
   const dim3 grid((unsigned)((tiles * gx + 7) / 8 * 8), calls), block(FWAVES * WAVE);
   const bool vx = p.K % 4 == 0 && (uintptr_t)p.a % (4 * sizeof(AT)) == 0 && p.a_cs % 4 == 0;
@@ -289,7 +302,11 @@ static void launch_float_tile(const FloatArgs &p, int rows, int max_active, int 
     else if (kf == K_QUADS) FLT_KF(RT_, K_QUADS);  \
     else FLT_KF(RT_, K_ANY);                       \
   } while (0)
-  if (rows == 16) FLT_RT(1);
+  if (p.N > F_MAX_N && rows == 16)
+    hipLaunchKernelGGL((k_float_tile<MODE, AT, WT, OT, 1, K_WIDE, 2>), grid, block, 0, s, p, gx);
+  else if (p.N > F_MAX_N)
+    hipLaunchKernelGGL((k_float_tile<MODE, AT, WT, OT, 2, K_WIDE, 2>), grid, block, 0, s, p, gx);
+  else if (rows == 16) FLT_RT(1);
   else FLT_RT(2);
 #undef FLT_RT
 #undef FLT_KF
@@ -308,9 +325,8 @@ int launch_float_expert(const FloatArgs &p, int mode, moe_dtype a_dt, moe_dtype 
     return moe_fail(MOE_INVALID_ARGUMENT, "float expert: K " + std::to_string(p.K) +
                                               " is too long for the 64 KB row stage");
   const int rows = float_tile_rows(p.db.A, max_active, w_dt);
-  if (((int64_t)p.db.A + max_active) * ((p.N + FCOLS - 1) / FCOLS) > 0x7ffffff0)
+  if (((int64_t)p.db.A + max_active) * (((int64_t)p.N + FCOLS - 1) / FCOLS) > 0x7ffffff0)
     return moe_fail(MOE_INVALID_ARGUMENT, "float expert: too many rows");
-  if (p.N > (1 << 24)) return moe_fail(MOE_INVALID_ARGUMENT, "float expert: more than 2^24 columns");
 #define FLT(M_, A_, W_, O_) launch_float_tile<M_, A_, W_, O_>(p, rows, max_active, calls, s)
   const bool af = a_dt == MOE_F16, wf = w_dt == MOE_F16, of = o_dt == MOE_F16;
   if (mode == MODE_UP) {

@@ -191,3 +191,28 @@ def test_float_tiles(dtype, M, K, N, E):
     eps = (16 + K / 16 + 10) * 2.0 ** -24
     bound = eps * mag + (2.0 ** -11 * np.abs(want) + 1e-7 if dtype == "f16" else 0.0) + 1e-30
     np.testing.assert_array_less(np.abs(got - want), bound)
+
+
+# Weight rows so wide that 16 of them pass 32-bit offsets: 16- and 32-row tiles,
+# K past a step, an infinity in an expert's first row.
+@pytest.mark.parametrize("dtype,M,K", [("f32", 3, 5), ("f16", 40, 3), ("f32", 15, 18)])
+def test_float_more_than_2p24_columns(dtype, M, K):
+    print(f"float columns {dtype} M={M} K={K}", flush=True)
+    E, N = 2, (1 << 24) + 36
+    td = torch.float16 if dtype == "f16" else torch.float32
+    g = torch.Generator(device=DEV).manual_seed(M)
+    a = torch.randn((M, K), generator=g, device=DEV).to(td)
+    w = torch.randn((E * K, N), generator=g, device=DEV).to(td)
+    w[K, 4] = float("inf")
+    idx = (torch.arange(M, device=DEV) % E).float()
+    got = rt.matmulGather(a, w, idx, {"bias": torch.zeros((E, N), device=DEV, dtype=td)})
+    for c in (slice(0, 70), slice(N // 2, N // 2 + 64), slice(N - 68, N)):
+        for e in range(E):
+            r, we = a[e::E].double(), w[e * K:(e + 1) * K, c].double()
+            want = torch.stack([r[:, k:k + 1] * we[k] for k in range(K)]).sum(0)
+            have, fin = got[e::E, c].double(), torch.isfinite(want)
+            assert torch.equal(have[~fin], want[~fin])
+            bound = (16 + 10) * 2.0 ** -24 * (r.abs() @ we.abs())[fin]
+            if dtype == "f16":
+                bound = bound + 2.0 ** -11 * want[fin].abs() + 1e-7
+            assert torch.all((have - want)[fin].abs() <= bound + 1e-30)
