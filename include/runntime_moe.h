@@ -264,7 +264,8 @@ MOE_API int moe_viterbi_decode(const double *start, const double *end, const dou
                                const float *log_probs, int T, int n, int32_t *path);
 /* Linear (src/core/nn/layers.ts:166-263): out [T, N] = x [T, K] · w [K, N]
  * + bias [N] (or NULL) + addend [T, N] (or NULL), all f32, w row-major
- * [in, out] (a quantized checkpoint weight dequantized once at load). */
+ * [in, out] (a quantized checkpoint weight dequantized once at load). out may
+ * be addend, or overlap the inputs (it then goes through the workspace). */
 MOE_API int moe_linear(moe_ctx *ctx, const float *x, const float *w, const float *bias,
                        const float *addend, int T, int K, int N, float *out);
 /* The attention core of the privacy filter's block (src/zoo/privacy-filter/

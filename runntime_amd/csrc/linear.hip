@@ -210,7 +210,19 @@ __global__ __launch_bounds__(64 * KW) void k_linear(const float *__restrict__ x,
   }
 }
 
+__global__ void k_copy(const float *__restrict__ from, float *__restrict__ to, size_t n) {
+  const size_t stride = (size_t)gridDim.x * blockDim.x;
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) to[i] = from[i];
+}
+
 }  // namespace
+
+int launch_copy(const float *from, float *to, size_t n, hipStream_t s) {
+  const size_t blocks = (n + 255) / 256;
+  hipLaunchKernelGGL(k_copy, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s, from,
+                     to, n);
+  return 0;
+}
 
 int launch_linear(const float *x, const float *w, const float *bias, const float *addend, float *y,
                   int T, int K, int N, hipStream_t s) {

@@ -1005,7 +1005,19 @@ extern "C" int moe_linear(moe_ctx *ctx, const float *x, const float *w, const fl
   if (rc) return rc;
   REQUIRE(T >= 1 && K >= 1 && N >= 1, "linear: T, K and N must be positive");
   REQUIRE(x && w && out, "linear: NULL tensor");
-  if ((rc = launch_linear(x, w, bias, addend, out, T, K, N, ctx->stream))) return rc;
+  // k_linear's blocks read all of a row of x and a column of w while others
+  // have written theirs: an out over one of its inputs is filled by way of the
+  // workspace. (addend at out itself is read where it is written.)
+  const size_t nout = (size_t)T * N;
+  auto over = [&](const float *p, size_t n) {
+    return p && (uintptr_t)p < (uintptr_t)(out + nout) && (uintptr_t)out < (uintptr_t)(p + n);
+  };
+  const bool aside = over(x, (size_t)T * K) || over(w, (size_t)K * N) || over(bias, N) ||
+                     (addend != out && over(addend, nout));
+  if (aside && (rc = moe_ws_ensure(ctx, nout * 4))) return rc;
+  float *y = aside ? (float *)ctx->ws : out;
+  if ((rc = launch_linear(x, w, bias, addend, y, T, K, N, ctx->stream))) return rc;
+  if (aside && (rc = launch_copy(y, out, nout, ctx->stream))) return rc;
   return after_launch("linear");
 }
 

@@ -75,6 +75,7 @@ struct WsPlan {
   }
 };
 
+int launch_copy(const float *from, float *to, size_t n, hipStream_t s);
 int moe_ws_ensure(moe_ctx *ctx, size_t bytes);
 
 // ------------------------------------------------------------ constants

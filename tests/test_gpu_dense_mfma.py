@@ -58,6 +58,28 @@ def test_linear_more_than_2p24_columns(T, K, N):
         assert torch.all(err <= (32 + 12) * 2.0 ** -24 * mag[fin] + 1e-30)
 
 
+@pytest.mark.parametrize("over", ["x", "addend", "w", "x shifted"])
+def test_linear_into_its_inputs(over):
+    """out over x (K = N), the addend, the weight (T = K), or rows below x's own:
+    the result of a separate out."""
+    print(f"linear into {over}", flush=True)
+    from runntime_amd import _lib
+    from runntime_amd.core import _ctx
+    T = K = N = 640
+    g = torch.Generator(device=DEV).manual_seed(9)
+    buf = torch.randn((T + 8, K), generator=g, device=DEV)
+    x = buf[:T]
+    w = torch.randn((K, N), generator=g, device=DEV)
+    a = torch.randn((T, N), generator=g, device=DEV)
+    want = Linear(K, N, w.clone()).forward(x, a)
+    out = {"x": x, "addend": a, "w": w, "x shifted": buf[8:]}[over]
+    torch.cuda.synchronize()
+    _lib.check(_lib.load().moe_linear(_ctx(x.device), x.data_ptr(), w.data_ptr(), None, a.data_ptr(),
+                                      T, K, N, out.data_ptr()))
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+
+
 def test_linear_keeps_infinities_in_their_rows():
     print("linear infinities", flush=True)
     x = np.ones((40, 20), np.float32)
