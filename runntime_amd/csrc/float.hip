@@ -264,12 +264,6 @@ int launch_idx_route(const float *idx, int M, float *route, hipStream_t s) {
   return 0;
 }
 
-// Rows of the row stage of former versions: a K past it stays refused.
-static bool float_k_ok(int K, int mode, bool small) {
-  const int fw = small ? 8 : 4, frc = small ? 2 : 4;
-  return (size_t)frc * K * 4 + (size_t)fw * (mode == MODE_UP ? 2 : 1) * frc * WAVE * 16 <= 64 * 1024;
-}
-
 // Rows per tile, from the rows an expert has on average (block of 640 × 640, E
 // 128, top-4, µs, 16- and 32-row tiles: f32 150 tokens 143, 147, 300 tokens
 // 156, 155, 500 tokens 192, 171; f16, whose tiles cost half the bytes, 500
@@ -321,9 +315,6 @@ int launch_float_expert(const FloatArgs &p, int mode, moe_dtype a_dt, moe_dtype 
   MOE_NONNULL(p.db.active);
   MOE_NONNULL(p.db.meta);
   if (mode == MODE_UP) MOE_NONNULL(p.w1);
-  if (!float_k_ok(p.K, mode, (long)p.db.A <= 2l * max_active))
-    return moe_fail(MOE_INVALID_ARGUMENT, "float expert: K " + std::to_string(p.K) +
-                                              " is too long for the 64 KB row stage");
   const int rows = float_tile_rows(p.db.A, max_active, w_dt);
   if (((int64_t)p.db.A + max_active) * (((int64_t)p.N + FCOLS - 1) / FCOLS) > 0x7ffffff0)
     return moe_fail(MOE_INVALID_ARGUMENT, "float expert: too many rows");

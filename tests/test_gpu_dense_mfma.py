@@ -215,6 +215,30 @@ def test_float_tiles(dtype, M, K, N, E):
     np.testing.assert_array_less(np.abs(got - want), bound)
 
 
+# K past what a block's rows would fill in LDS (none are kept there): up and down,
+# one row an expert and many, at d and I of 4100.
+@pytest.mark.parametrize("T", [2, 40])
+def test_float_block_of_long_rows(T):
+    print(f"float block long rows T={T}", flush=True)
+    from tests.helpers import assert_close
+    d, I, E, k = 4100, 4100, 4, 2
+    rng = np.random.default_rng(T)
+    x = rng.standard_normal((T, d)).astype(np.float32)
+    norm = np.ones(d, np.float32)
+    rw = (0.02 * rng.standard_normal((d, E))).astype(np.float32)
+    rb = np.zeros(E, np.float32)
+    mk = lambda n, m, s: (s * rng.standard_normal((E * n, m))).astype(np.float32)
+    glu, lin, down = mk(d, I, d ** -0.5), mk(d, I, d ** -0.5), mk(I, d, I ** -0.5)
+    zi, zd = np.zeros((E, I), np.float32), np.zeros((E, d), np.float32)
+    out, route = rt.moe_block_float(_dev(x), _dev(norm), 1e-5, _dev(rw), _dev(rb), _dev(glu), _dev(zi),
+                                    _dev(lin), _dev(zi), _dev(down), _dev(zd), k=k, return_route=True)
+    xn = ref.rmsnorm(x, norm, 1e-5)
+    want_route = ref.topk(ref.router_logits(xn, rw, rb), k)
+    assert np.array_equal(route.cpu().numpy()[:, :k], want_route[:, :k])
+    want = ref.moe_block_float_f64(x, xn, want_route, (glu, zi), (lin, zi), (down, zd), k)
+    assert_close(out.cpu().numpy(), want, atol=1e-4, rtol=1e-4, what="long rows")
+
+
 # Weight rows so wide that 16 of them pass 32-bit offsets: 16- and 32-row tiles,
 # K past a step, an infinity in an expert's first row.
 @pytest.mark.parametrize("dtype,M,K", [("f32", 3, 5), ("f16", 40, 3), ("f32", 15, 18)])
