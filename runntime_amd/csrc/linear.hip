@@ -229,8 +229,6 @@ int launch_linear(const float *x, const float *w, const float *bias, const float
   MOE_NONNULL(x);
   MOE_NONNULL(w);
   MOE_NONNULL(y);
-  if ((T + 15) / 16 > 65535)
-    return moe_fail(MOE_INVALID_ARGUMENT, "linear: more than " + std::to_string(65535 * 16) + " rows");
   auto aligned = [](const void *p, int bytes) { return (uintptr_t)p % bytes == 0; };
   const bool vx = K % 4 == 0 && aligned(x, 16);
   auto cols_ok = [&](int ct) {

@@ -58,6 +58,20 @@ def test_linear_more_than_2p24_columns(T, K, N):
         assert torch.all(err <= (32 + 12) * 2.0 ** -24 * mag[fin] + 1e-30)
 
 
+@pytest.mark.parametrize("K,N", [(16, 64), (3, 1)])
+def test_linear_past_65535_row_tiles(K, N):
+    T = 65535 * 32 + 33
+    print(f"linear T={T} K={K} N={N}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(K)
+    x = torch.randn((T, K), generator=g, device=DEV)
+    w = torch.randn((K, N), generator=g, device=DEV)
+    got = Linear(K, N, w).forward(x)
+    for r in (slice(0, 40), slice(65535 * 16 - 20, 65535 * 16 + 20), slice(T - 40, T)):
+        xr = x[r].double()
+        err = (got[r].double() - xr @ w.double()).abs()
+        assert torch.all(err <= (32 + 12) * 2.0 ** -24 * (xr.abs() @ w.double().abs()) + 1e-30)
+
+
 @pytest.mark.parametrize("over", ["x", "addend", "w", "x shifted"])
 def test_linear_into_its_inputs(over):
     """out over x (K = N), the addend, the weight (T = K), or rows below x's own:
