@@ -79,13 +79,14 @@ __global__ __launch_bounds__(64 * KW) void k_linear(const float *__restrict__ x,
                                                     const float *__restrict__ bias,
                                                     const float *__restrict__ addend,
                                                     float *__restrict__ y, int T, int K, int N,
-                                                    int ncb) {
+                                                    int ncb, int blk0) {
   typedef typename Cols<CT>::type colv;
   constexpr int PD = RT == 1 ? 4 : 2;  // steps loaded (this one and those ahead)
   __shared__ colv red[KW][RT * 4][WAVE];
   const int lane = threadIdx.x & (WAVE - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-  const int rb = blockIdx.x / ncb, cb = blockIdx.x - rb * ncb;
+  const int blk = blk0 + (int)blockIdx.x;
+  const int rb = blk / ncb, cb = blk - rb * ncb;
   const int row0 = rb * 16 * RT, col0 = cb * 16 * CT;
   const int m = lane & 15, kq = lane >> 4;
   const int steps = (K + LSTEP - 1) / LSTEP;
@@ -249,9 +250,13 @@ int launch_linear(const float *x, const float *w, const float *bias, const float
   const int64_t n = blocks(rt, ct);
   if (n > 0x7fffffff) return moe_fail(MOE_INVALID_ARGUMENT, "linear: output too large");
   const int ncb = (int)(((int64_t)N + 16 * ct - 1) / (16 * ct));
+  // A grid holds fewer than 2^32 threads: larger outputs in several launches.
+  if (T > 0x7fffffc0) return moe_fail(MOE_INVALID_ARGUMENT, "linear: output too large");
+  constexpr int64_t GRID = 1 << 22;
 #define LIN_KF(RT_, CT_, KW_, KF_)                                                                \
-  hipLaunchKernelGGL((k_linear<RT_, CT_, KW_, KF_>), dim3((unsigned)n), dim3(64 * KW_), 0, s, x, w, \
-                     bias, addend, y, T, K, N, ncb)
+  for (int64_t b = 0; b < n; b += GRID)                                                           \
+  hipLaunchKernelGGL((k_linear<RT_, CT_, KW_, KF_>), dim3((unsigned)(n - b < GRID ? n - b : GRID)), \
+                     dim3(64 * KW_), 0, s, x, w, bias, addend, y, T, K, N, ncb, (int)b)
 #define LIN(RT_, CT_, KW_)                                   \
   do {                                                       \
     if (K % LSTEP == 0) LIN_KF(RT_, CT_, KW_, K_STEPS);      \

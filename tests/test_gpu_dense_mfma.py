@@ -58,9 +58,11 @@ def test_linear_more_than_2p24_columns(T, K, N):
         assert torch.all(err <= (32 + 12) * 2.0 ** -24 * mag[fin] + 1e-30)
 
 
-@pytest.mark.parametrize("K,N", [(16, 64), (3, 1)])
-def test_linear_past_65535_row_tiles(K, N):
-    T = 65535 * 32 + 33
+# Row tiles past a grid's second dimension, and outputs of more blocks than one
+# grid holds threads for (16 x 16 tiles of 2^31 outputs and more).
+@pytest.mark.parametrize("T,K,N", [(65535 * 32 + 33, 16, 64), (65535 * 32 + 33, 3, 1),
+                                   (1050001, 1, 2047)])
+def test_linear_many_rows(T, K, N):
     print(f"linear T={T} K={K} N={N}", flush=True)
     g = torch.Generator(device=DEV).manual_seed(K)
     x = torch.randn((T, K), generator=g, device=DEV)
