@@ -84,7 +84,7 @@ enum KForm { K_STEPS = 0, K_QUADS = 1, K_ANY = 2, K_WIDE = 3 };
 constexpr int F_MAX_N = 1 << 24;
 // FPD: steps loaded (the one multiplied and those ahead of it).
 template <int MODE, typename AT, typename WT, typename OT, int RT, int KF, int FPD>
-__global__ __launch_bounds__(FWAVES *WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_float_tile(FloatArgs p, int gx) {
+__global__ __launch_bounds__(FWAVES *WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_float_tile(FloatArgs p, int gx, int blk0) {
   constexpr int NS = MODE == MODE_UP ? 2 : 1;
   constexpr int KW = FWAVES / NS;           // wavefronts per weight array
   constexpr int ROWS = 16 * RT;
@@ -104,8 +104,9 @@ __global__ __launch_bounds__(FWAVES *WAVE) __attribute__((amdgpu_waves_per_eu(4)
   const int na = meta[META_ACTIVE];
   const int total = meta[META_TILES] * gx;
   const int per = (total + 7) / 8;
-  const int slot = blockIdx.x >> 3;
-  const int o = (blockIdx.x & 7) * per + slot;
+  const int blk = blk0 + (int)blockIdx.x;  // blk0 a multiple of 8
+  const int slot = blk >> 3;
+  const int o = (blk & 7) * per + slot;
   if (slot >= per || o >= total) return;
   const int mt = o / gx, xb = o - mt * gx;
   int hit = __popcll(__ballot(lane < na && ad.w <= mt)) - 1;
@@ -276,7 +277,10 @@ template <int MODE, typename AT, typename WT, typename OT>
 static void launch_float_tile(const FloatArgs &p, int rows, int max_active, int calls, hipStream_t s) {
   const int gx = (int)(((int64_t)p.N + FCOLS - 1) / FCOLS);
   const int64_t tiles = (int64_t)(p.db.A - max_active) / rows + max_active;
-  const dim3 grid((unsigned)((tiles * gx + 7) / 8 * 8), calls), block(FWAVES * WAVE);
+  // A grid holds fewer than 2^32 threads: larger outputs in several launches.
+  const int64_t nblk = (tiles * gx + 7) / 8 * 8;
+  constexpr int64_t GRID = 1 << 22;
+  const dim3 block(FWAVES * WAVE);
   const bool vx = p.K % 4 == 0 && (uintptr_t)p.a % (4 * sizeof(AT)) == 0 && p.a_cs % 4 == 0;
   const int kf = !vx ? K_ANY : p.K % FSTEP ? K_QUADS : K_STEPS;
   // 16-row tiles that fill the CUs twice: no step ahead, the registers for
@@ -286,9 +290,9 @@ static void launch_float_tile(const FloatArgs &p, int rows, int max_active, int 
 #define FLT_KF(RT_, KF_)                                                                            \
   do {                                                                                              \
     if (RT_ == 1 && full)                                                                           \
-      hipLaunchKernelGGL((k_float_tile<MODE, AT, WT, OT, RT_, KF_, 1>), grid, block, 0, s, p, gx);  \
+      hipLaunchKernelGGL((k_float_tile<MODE, AT, WT, OT, RT_, KF_, 1>), grid, block, 0, s, p, gx, (int)b);  \
     else                                                                                            \
-      hipLaunchKernelGGL((k_float_tile<MODE, AT, WT, OT, RT_, KF_, 2>), grid, block, 0, s, p, gx);  \
+      hipLaunchKernelGGL((k_float_tile<MODE, AT, WT, OT, RT_, KF_, 2>), grid, block, 0, s, p, gx, (int)b);  \
   } while (0)
 #define FLT_RT(RT_)                                \
   do {                                             \
@@ -296,12 +300,17 @@ static void launch_float_tile(const FloatArgs &p, int rows, int max_active, int 
     else if (kf == K_QUADS) FLT_KF(RT_, K_QUADS);  \
     else FLT_KF(RT_, K_ANY);                       \
   } while (0)
-  if (p.N > F_MAX_N && rows == 16)
-    hipLaunchKernelGGL((k_float_tile<MODE, AT, WT, OT, 1, K_WIDE, 2>), grid, block, 0, s, p, gx);
-  else if (p.N > F_MAX_N)
-    hipLaunchKernelGGL((k_float_tile<MODE, AT, WT, OT, 2, K_WIDE, 2>), grid, block, 0, s, p, gx);
-  else if (rows == 16) FLT_RT(1);
-  else FLT_RT(2);
+  for (int64_t b = 0; b < nblk; b += GRID) {
+    const dim3 grid((unsigned)(nblk - b < GRID ? nblk - b : GRID), calls);
+    if (p.N > F_MAX_N && rows == 16)
+      hipLaunchKernelGGL((k_float_tile<MODE, AT, WT, OT, 1, K_WIDE, 2>), grid, block, 0, s, p, gx,
+                         (int)b);
+    else if (p.N > F_MAX_N)
+      hipLaunchKernelGGL((k_float_tile<MODE, AT, WT, OT, 2, K_WIDE, 2>), grid, block, 0, s, p, gx,
+                         (int)b);
+    else if (rows == 16) FLT_RT(1);
+    else FLT_RT(2);
+  }
 #undef FLT_RT
 #undef FLT_KF
 }

@@ -278,3 +278,16 @@ def test_float_more_than_2p24_columns(dtype, M, K):
             if dtype == "f16":
                 bound = bound + 2.0 ** -11 * want[fin].abs() + 1e-7
             assert torch.all((have - want)[fin].abs() <= bound + 1e-30)
+
+
+def test_float_more_outputs_than_a_grid():
+    """Past 2^34 outputs, 32-row tiles of 64 columns and eight wavefronts are more
+    threads than one grid holds."""
+    M, N = (1 << 22) + 40, 4096
+    print(f"float outputs {M} x {N}", flush=True)
+    a = ((torch.arange(M, device=DEV) % 1021) - 510).to(torch.float16).reshape(M, 1)
+    w = ((torch.arange(N, device=DEV) % 7) - 3).to(torch.float16).reshape(1, N)
+    got = rt.matmulGather(a, w, torch.zeros(M, device=DEV),
+                          {"bias": torch.zeros((1, N), device=DEV, dtype=torch.float16)})
+    for r in range(0, M, 1 << 20):
+        assert torch.equal(got[r:r + (1 << 20)], a[r:r + (1 << 20)] * w), r
