@@ -317,9 +317,11 @@ typedef struct moe_call_strides {
 /* `calls` independent moe_layer calls of identical shape, enqueued as one
  * set of kernels: call c reads and writes every tensor at
  * base + c·stride (strides NULL: all 0, valid for calls == 1). Each call is
- * routed, dispatched and computed on its own, exactly as moe_layer would;
- * the calls only share the launches. x, out and route_out need non-zero
- * strides when calls > 1. No reference counterpart: it lets single-token
+ * routed, dispatched and computed on its own, with moe_layer's route bit for
+ * bit and its outputs but for f32 rounding: the kernels and their splits of K
+ * are chosen for the work of all calls (moe_expert_tiles), and sum in another
+ * order where that differs from one call's. x, out and route_out need
+ * non-zero strides when calls > 1. No reference counterpart: it lets single-token
  * decode calls of separate layer instances (e.g. independent requests on
  * separate weight sets) fill the GPU instead of running one launch-bound
  * call at a time. */

@@ -14,7 +14,7 @@ import runntime_amd as rt
 from oracle import ref
 from runntime_amd.quantw import QuantExpertWeight, QuantW
 from runntime_amd.synth import CONFIGS, make_inputs
-from tests.helpers import assert_close, random_quant_weight, route_for
+from tests.helpers import assert_close, expert_tiles, random_quant_weight, route_for
 
 pytestmark = pytest.mark.gpu
 
@@ -478,8 +478,9 @@ def _slice_weight(w, c):
 @pytest.mark.parametrize("T,cfg_id", [(1, 2), (5, 1), (40, 1)])
 def test_moe_layer_batched_equals_single_calls(T, cfg_id):
     """Each call of a batch is the same computation as a standalone
-    moe_layer call on that call's slices (bit for bit), and the first call
-    matches the oracle."""
+    moe_layer call on that call's slices (bit for bit while both take the same
+    kernels and splits of K, as these do), and the first call matches the
+    oracle."""
     from runntime_amd.synth import make_weight_copies
     cfg = CONFIGS[cfg_id]
     C = 3
@@ -511,6 +512,38 @@ def test_moe_layer_batched_equals_single_calls(T, cfg_id):
     act = ref.moe_up(xs, want_route, wt(wc.glu), wt(wc.lin), 8, cfg.d, cfg.E)
     want = ref.moe_down(act, want_route, wt(wc.down), res[0].numpy(), 8, cfg.I, cfg.E)
     assert_close(out[0], want, what="batched call 0")
+
+
+def test_moe_layer_batched_on_other_kernels_than_one_call():
+    """Six calls of five tokens have the wavefronts for the row tiles, one call
+    takes the decode kernels: routes bit for bit, outputs against the oracle and
+    within f32 rounding of the single call's."""
+    from runntime_amd.synth import MoeConfig, make_weight_copies
+    cfg = MoeConfig("batched6", 5, 512, 8, 2, 1024, "f32")
+    C = 6
+    say(f"moe_layer_batched calls={C} {cfg}")
+    assert expert_tiles("layer", cfg.T, cfg.d, cfg.I, cfg.E, cfg.k, "f32") == (0, 0)
+    assert expert_tiles("layer", cfg.T, cfg.d, cfg.I, cfg.E, cfg.k, "f32", calls=C) == (16, 16)
+    wc = make_weight_copies(cfg, C, seed=15, device="cpu")
+    g = torch.Generator().manual_seed(13)
+    x = torch.randn((C, cfg.T, cfg.d), generator=g)
+    res = torch.randn((C, cfg.T, cfg.d), generator=g)
+    dev = lambda t: t.to(DEV)
+    dw = lambda w: QuantExpertWeight(QuantW(dev(w.w.words), w.w.dims), dev(w.scales), dev(w.bias))
+    out, route = rt.moe_layer_batched(dev(x), dev(wc.router_w), dev(wc.router_b), dw(wc.glu),
+                                      dw(wc.lin), dw(wc.down), dev(res), cfg.k)
+    out, route = host(out), host(route)
+    for c in range(C):
+        o1, r1 = rt.moe_layer(dev(x[c]), dev(wc.router_w[c]), dev(wc.router_b[c]),
+                              dw(_slice_weight(wc.glu, c)), dw(_slice_weight(wc.lin, c)),
+                              dw(_slice_weight(wc.down, c)), dev(res[c]), cfg.k, return_route=True)
+        assert np.array_equal(host(r1), route[c])
+        wt = lambda w: (w.w.words[c].numpy().view(np.uint32), w.scales[c].numpy(), w.bias[c].numpy())
+        act = ref.moe_up(x[c].numpy(), route[c], wt(wc.glu), wt(wc.lin), 8, cfg.d, cfg.E)
+        want = ref.moe_down(act, route[c], wt(wc.down), res[c].numpy(), 8, cfg.I, cfg.E)
+        assert_close(out[c], want, what=f"batched call {c}")
+        # both sides within about 2^-20 of f64 each (norm over norm)
+        assert np.linalg.norm(out[c] - host(o1)) <= 2.0 ** -19 * np.linalg.norm(want)
 
 
 def test_moe_layer_batched_config3_shape():
