@@ -22,7 +22,7 @@ def _dev(a):
 # K of one step, past a step by 4 and by 1, fewer steps than wavefronts.
 @pytest.mark.parametrize("T,K,N", [(1, 16, 1), (17, 20, 33), (16, 640, 64), (65, 640, 1152),
                                    (31, 132, 70), (321, 896, 644), (1000, 24, 260), (700, 647, 66),
-                                   (160, 33, 1600)])
+                                   (160, 33, 1600), (65, 132, 1150)])
 def test_linear_tiles(T, K, N):
     print(f"linear T={T} K={K} N={N}", flush=True)
     rng = np.random.default_rng(T + N)
@@ -113,7 +113,9 @@ ATTN = [  # q_len, kv_len, q_heads, kv_heads, head_dim, left, right, offset, ext
     (15, 15, 14, 2, 64, 128, 128, 0, "sinks"), (17, 33, 3, 1, 128, 5, 0, 16, "sinks"),
     (33, 64, 8, 1, 64, 0, 0, 31, ""), (64, 64, 4, 2, 128, 40, 40, 0, "segments"),
     (97, 97, 9, 1, 64, 31, 7, 0, "segments sinks"), (50, 200, 2, 1, 64, -1, -1, 0, "bias"),
-    (300, 300, 16, 2, 64, 128, 128, 0, "sinks"), (700, 700, 18, 2, 64, 30, 30, 0, "sinks")]
+    (300, 300, 16, 2, 64, 128, 128, 0, "sinks"), (700, 700, 18, 2, 64, 30, 30, 0, "sinks"),
+    # eight heads a block, the second block of a kv head with one of nine
+    (500, 500, 72, 8, 64, 9, 3, 0, "segments sinks")]
 
 
 @pytest.mark.parametrize("dtype", ["f32", "f16"])
@@ -207,10 +209,12 @@ def test_sdpa_keeps_infinities_from_rows_that_do_not_see_them(dtype, n, qh, kh, 
 
 
 # Rows per expert from one to a second 32-row tile; K whole steps, past one by
-# 4, and odd; N a partial column block; many blocks (no step ahead) and few.
+# 4, and odd; N a partial column block; few blocks, and 16-row tiles of 512 and
+# more (no step ahead).
 @pytest.mark.parametrize("dtype", ["f32", "f16"])
 @pytest.mark.parametrize("M,K,N,E", [(1, 16, 4, 1), (33, 36, 68, 2), (200, 640, 132, 40),
-                                     (130, 19, 64, 3), (90, 48, 260, 90), (700, 260, 72, 16)])
+                                     (130, 19, 64, 3), (90, 48, 260, 90), (700, 260, 72, 16),
+                                     (120, 640, 260, 120), (120, 260, 260, 120), (120, 19, 260, 120)])
 def test_float_tiles(dtype, M, K, N, E):
     print(f"float tiles {dtype} M={M} K={K} N={N} E={E}", flush=True)
     rng = np.random.default_rng(M + K)

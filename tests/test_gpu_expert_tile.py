@@ -10,17 +10,23 @@ import runntime_amd as rt
 from oracle import ref
 
 from runntime_amd.synth import MoeConfig, make_inputs
-from tests.helpers import assert_close, random_quant_weight
+from tests.helpers import assert_close, expert_tiles, random_quant_weight
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
-# (T, K, N, E, g, k): rows per expert from 1 to a second 64-row tile, K one
-# 32-wide step past a piece or a ring turn, N with a partial unit group, a
-# partial column block and a wavefront without columns.
+# (T, K, N, E, g, k), rows per tile: rows per expert from 1 to many 16-row tiles
+# (a launch of fewer than 512 blocks takes no larger ones), then row tiles of 32
+# and 64; K one 32-wide step past a piece or a ring turn or a part of a step, N
+# with a partial unit group, a partial column block and a wavefront without
+# columns.
 SHAPES = [(1, 32, 8, 3, 32, 2), (5, 96, 72, 4, 32, 2), (40, 160, 136, 8, 32, 2),
           (60, 288, 264, 6, 96, 2), (129, 640, 200, 4, 640, 2), (70, 352, 64, 2, 352, 1),
           (260, 416, 520, 4, 416, 1), (33, 1408, 68, 1, 64, 1), (90, 64, 640, 128, 64, 4)]
+LARGE = [((160, 104, 1416, 32, 104, 4), 32), ((160, 160, 1416, 32, 32, 4), 32),
+         ((160, 288, 1352, 32, 96, 4), 32), ((320, 104, 1416, 32, 104, 4), 64),
+         ((320, 160, 1416, 32, 32, 4), 64), ((320, 288, 1352, 32, 288, 4), 64)]
+TILES = [(c, 0 if c[0] == 1 else 16) for c in SHAPES] + LARGE
 
 
 def _route(T, E, k, seed):
@@ -56,9 +62,13 @@ def _project(x, ids, w, b):
 
 @pytest.mark.parametrize("bits", [8, 4])
 @pytest.mark.parametrize("xdtype", ["f32", "f16"])
-@pytest.mark.parametrize("shape", SHAPES)
-def test_tile_products(bits, xdtype, shape):
+@pytest.mark.parametrize("shape,rows", TILES)
+def test_tile_products(bits, xdtype, shape, rows):
     T, K, N, E, g, k = shape
+    if bits == 4:  # int4 runs here from one row on
+        rows = max(rows, 16)
+    assert expert_tiles("up", T, K, N, E, k, xdtype, bits, g, g)[0] == rows
+    assert expert_tiles("down", T, N, K, E, k, "f32", bits, g, g)[1] == rows
     print(f"expert tile int{bits} {xdtype} {shape}", flush=True)
     route = _route(T, E, k, T + K)
     ids = route[:, :k].reshape(-1)
@@ -156,36 +166,46 @@ def test_experts_of_half_a_gib(bits, K, N, T):
             assert torch.all((got - want).abs() <= bound), (u, e)
 
 
-# Layers on each side of the rules: few rows per expert on wide weights, row
-# tiles of 16, 32 and 64, K not a multiple of 32 (I = 1000), and the grouped
-# GEMM's forms from 80 (f16 x: int8 limbs, an odd number of step pairs; f16
-# pairs when I is not a multiple of 64) and 64 (f32 x) rows per expert.
-LAYERS = [MoeConfig("t_wide3", 3, 1024, 16, 4, 2816, "f16"),
-          MoeConfig("t_rows5", 40, 640, 32, 4, 640, "f32"),
-          MoeConfig("t_rows20_i1000", 160, 768, 32, 4, 1000, "f16"),
-          MoeConfig("t_rows40", 320, 640, 32, 4, 640, "f32"),
-          MoeConfig("t_skew", 512, 640, 16, 2, 384, "f16", zipf=1.2, hot_share=0.5, empty=2),
-          MoeConfig("g_limbs_odd", 300, 1024, 6, 2, 1088, "f16"),
-          MoeConfig("g_pairs_i1056", 300, 1024, 6, 2, 1056, "f16"),
-          MoeConfig("g_f32x", 300, 640, 6, 2, 640, "f32")]
+# Layers on each side of the rules, and the rows per tile of both products: few
+# rows per expert on wide weights (decode kernels), row tiles of 16, 32 and 64
+# (from 32 on the dispatch counts in them), K not a multiple of 32 (I = 1000), and
+# the grouped GEMM's forms (f16 x: int8 limbs, an odd number of step pairs; f16
+# pairs when I is not a multiple of 64; f32 x).
+LAYERS = [(MoeConfig("t_wide3", 3, 1024, 16, 4, 2816, "f16"), 0),
+          (MoeConfig("t_rows5", 40, 640, 32, 4, 640, "f32"), 16),
+          (MoeConfig("t_rows20_i1000", 160, 768, 32, 4, 1000, "f16"), 16),
+          (MoeConfig("t_rows40", 320, 640, 32, 4, 640, "f32"), 16),
+          (MoeConfig("t_skew", 512, 640, 16, 2, 384, "f16", zipf=1.2, hot_share=0.5, empty=2), 16),
+          (MoeConfig("t_limbs_odd", 300, 1024, 6, 2, 1088, "f16"), 16),
+          (MoeConfig("t_rows20", 160, 256, 32, 4, 1408, "f16"), 32),
+          (MoeConfig("t_rows20_f32", 160, 256, 32, 4, 1416, "f32"), 32),
+          (MoeConfig("t_rows40_wide", 320, 256, 32, 4, 1408, "f16"), 64),
+          (MoeConfig("t_rows40_f32", 320, 256, 32, 4, 1416, "f32"), 64),
+          (MoeConfig("t_skew64", 320, 256, 32, 4, 1408, "f16", zipf=1.2, hot_share=0.5, empty=2), 64),
+          (MoeConfig("g_limbs_odd", 1000, 1024, 20, 2, 1088, "f16"), 128),
+          (MoeConfig("g_pairs_i1056", 1024, 1024, 8, 2, 1056, "f16"), 128),
+          (MoeConfig("g_f32x", 1536, 1024, 8, 2, 1024, "f32"), 128)]
+CHECKED = 150  # tokens checked against the oracle, spread over the call
 
 
-@pytest.mark.parametrize("cfg", LAYERS, ids=[c.name for c in LAYERS])
-def test_layer_paths(cfg):
+@pytest.mark.parametrize("cfg,rows", LAYERS, ids=[c.name for c, _ in LAYERS])
+def test_layer_paths(cfg, rows):
     print(f"layer path {cfg}", flush=True)
+    assert expert_tiles("layer", cfg.T, cfg.d, cfg.I, cfg.E, cfg.k, cfg.x_dtype) == (rows, rows)
     inp = make_inputs(cfg, seed=12, keep_q=True, bias_rand=True)
     inp.residual.copy_(torch.randn(tuple(inp.residual.shape), generator=torch.Generator().manual_seed(6)))
     out, route = rt.moe_layer(inp.x, inp.router_w, inp.router_b, inp.glu, inp.lin, inp.down,
                               inp.residual, cfg.k, return_route=True)
-    x = inp.x.float().cpu().numpy()
+    t = np.unique(np.linspace(0, cfg.T - 1, CHECKED).astype(int)) if cfg.T > 512 else np.arange(cfg.T)
+    x = inp.x[t].float().cpu().numpy()
     want_route = ref.topk(ref.router_logits(x, inp.router_w.cpu().numpy(),
                                             inp.router_b.cpu().numpy()), cfg.k)
     w = {n: (ref.pack_ekn(inp.q[n].numpy(), 8), getattr(inp, n).scales.cpu().numpy(),
              getattr(inp, n).bias.cpu().numpy()) for n in ("glu", "lin", "down")}
     act = ref.moe_up(x, want_route, w["glu"], w["lin"], 8, cfg.d, cfg.E)
-    want = ref.moe_down(act, want_route, w["down"], inp.residual.cpu().numpy(), 8, cfg.I, cfg.E)
-    assert np.array_equal(route.cpu().numpy()[:, :cfg.k], want_route[:, :cfg.k])
-    assert_close(out.cpu().numpy(), want, what=cfg.name)
+    want = ref.moe_down(act, want_route, w["down"], inp.residual[t].cpu().numpy(), 8, cfg.I, cfg.E)
+    assert np.array_equal(route.cpu().numpy()[t, :cfg.k], want_route[:, :cfg.k])
+    assert_close(out.cpu().numpy()[t], want, what=cfg.name)
 
 
 # Dispatch over the routes of each sort kernel: one block (1, 2, 4 and 8

@@ -14,7 +14,7 @@ import torch
 import runntime_amd as rt
 from oracle import ref
 from runntime_amd.synth import CONFIGS, make_inputs
-from tests.helpers import assert_close
+from tests.helpers import assert_close, expert_tiles
 from tests.test_gpu_parity import _edge_tokens
 from tests.test_oracle_norm import OPTIONS, SHAPES, inputs
 
@@ -158,17 +158,22 @@ def test_moe_block_is_norm_then_layer(cid, T, x_dtype):
     assert np.array_equal(host(out), host(o2))
 
 
-@pytest.mark.parametrize("T,d,x_dtype", [(33, 200, "f16"), (10, 2304, None)])
-def test_moe_block_staged_norm_row_lengths(T, d, x_dtype):
-    """The router's staged pre-norm reads a wavefront's rows together for
-    rows of up to 2048 elements (shorter rows in fewer loads per lane) and
-    row by row beyond; both stay bit-identical to rmsNorm → moe_layer. T = 33
-    leaves the last token tile one token, so most wavefronts have none."""
+@pytest.mark.parametrize("T,d,x_dtype,rows", [(33, 200, "f16", 16), (10, 2304, None, 16),
+                                              (2, 200, "f16", 0), (5, 200, "f32", 0),
+                                              (3, 2304, None, 0), (5, 2304, "f16", 0)])
+def test_moe_block_staged_norm_row_lengths(T, d, x_dtype, rows):
+    """A few rows an expert (rows 0: the decode kernels) take the pre-norm staged
+    by the router and the gate/up kernel, more the row tiles with a normalised
+    copy. The router reads a wavefront's rows together for rows of up to 2048
+    elements (shorter rows in fewer loads per lane) and row by row beyond. All
+    stay bit-identical to rmsNorm → moe_layer. T = 33 leaves the last token tile
+    one token, so most wavefronts have none."""
     import dataclasses
     cfg = dataclasses.replace(CONFIGS[3], T=T, d=d, E=16, I=256)
     if x_dtype:
         cfg = dataclasses.replace(cfg, x_dtype=x_dtype)
     say(f"moe_block staged norm T={T} d={d} {cfg.x_dtype}")
+    assert expert_tiles("layer", T, d, cfg.I, cfg.E, cfg.k, cfg.x_dtype) == (rows, rows)
     inp = make_inputs(cfg, seed=40 + d, bias_rand=True)
     nw = _norm_weight(cfg.d, cfg.x_dtype, 9).to(DEV)
     out, route = rt.moe_block(inp.x, nw, 1e-5, inp.router_w, inp.router_b, inp.glu, inp.lin,

@@ -153,7 +153,17 @@ MFMA_SHAPES = [(3, 64, 72, 5, 64), (40, 96, 136, 6, 32), (100, 100, 80, 3, 100),
                (17, 2048, 1408, 4, 2048), (64, 512, 1024, 8, 512), (9, 640, 640, 16, 64)]
 
 
-def _check_up(T, K, N, E, g, bits, k=4, xdtype="f32", tol="ref", route=None):
+def _checked(route, E, k, sample):
+    """All tokens, or `sample` of them spread evenly and those at the edges of
+    row tiles (tokens are independent of each other)."""
+    T = len(route)
+    if sample is None:
+        return np.arange(T)
+    return np.array(sorted(set(np.linspace(0, T - 1, sample).astype(int).tolist()) |
+                           _edge_tokens(route[:, :k], E, k)))
+
+
+def _check_up(T, K, N, E, g, bits, k=4, xdtype="f32", tol="ref", route=None, sample=None):
     route = route_for(T, E, k) if route is None else route
     glu, glu_h = weight_pair(E, K, N, bits, g, 10)
     lin, lin_h = weight_pair(E, K, N, bits, g, 20)
@@ -162,19 +172,23 @@ def _check_up(T, K, N, E, g, bits, k=4, xdtype="f32", tol="ref", route=None):
         x = x.astype(np.float16).astype(np.float32)
     xt = gpu(x, torch.float16 if xdtype == "f16" else torch.float32)
     got = host(rt.moeUp(xt, gpu(route), glu, lin, {"bits": bits, "groupSize": g}))
-    want = ref.moe_up(x, route, glu_h, lin_h, bits, g, E)
+    t = _checked(route, E, k, sample)
+    got = got.reshape(T, k, N)[t].reshape(-1, N)
+    want = ref.moe_up(x[t], route[t], glu_h, lin_h, bits, g, E)
     if tol == "ref":
         np.testing.assert_allclose(got, want, atol=1e-5 * K, rtol=1e-4)
     assert_close(got, want, what="moeUp")
 
 
-def _check_down(T, K, N, E, g, bits, k=4, route=None):
+def _check_down(T, K, N, E, g, bits, k=4, route=None, sample=None):
     route = route_for(T, E, k) if route is None else route
     down, down_h = weight_pair(E, K, N, bits, g, 30)
     act = ref.lcg_f32(T * k * K, 1).reshape(T * k, K)
     res = ref.lcg_f32(T * N, 4).reshape(T, N)
     got = host(rt.moeDown(gpu(act), gpu(route), down, gpu(res), {"bits": bits, "groupSize": g}))
-    want = ref.moe_down(act, route, down_h, res, bits, g, E)
+    t = _checked(route, E, k, sample)
+    got = got[t]
+    want = ref.moe_down(act.reshape(T, k, K)[t].reshape(-1, K), route[t], down_h, res[t], bits, g, E)
     np.testing.assert_allclose(got, want, atol=1e-5 * K, rtol=1e-4)
     assert_close(got, want, what="moeDown")
 
@@ -216,34 +230,52 @@ def test_moe_down_mfma(shape, k):
     _check_down(T, K, N, E, g, 8, k=k)
 
 
-# Rows per expert ≥ 64 on average: shapes for the grouped GEMM path. The
-# first list keeps K short, below the GEMM's load ring (≥ 18 steps of 32 for
-# f16 input, ≥ 12 for f32), so most of it runs the skinny kernel on many rows.
+# 64 rows an expert and more on few tiles: the row-tile kernel (16- and 32-row
+# tiles; 64 in down), but for the second of GEMM_UP_SHAPES with f16 x.
 GEMM_SHAPES = [(300, 128, 256, 4, 128), (260, 192, 128, 3, 192), (1000, 256, 384, 8, 256),
                (2048, 512, 640, 16, 512)]
-# These take the grouped GEMM: ragged last M-tiles, an N-tile with only part
-# of its units (N not a multiple of 256 / 512, and I = 1408's half tile),
-# the shortest K the ring takes.
 GEMM_UP_SHAPES = [(300, 640, 264, 4, 640), (1000, 768, 1408, 8, 768), (2048, 576, 640, 16, 576),
                   (600, 384, 136, 3, 384)]
-# Down: the last two split K into two partial products (few tiles for the
-# CUs), added by the combine.
 GEMM_DOWN_SHAPES = [(300, 384, 520, 4, 384), (1000, 1408, 2048, 8, 1408), (512, 5632, 256, 4, 5632)]
 
 
 @pytest.mark.parametrize("xdtype", ["f32", "f16"])
 @pytest.mark.parametrize("shape", GEMM_SHAPES + GEMM_UP_SHAPES)
-def test_moe_up_grouped_gemm(xdtype, shape):
+def test_moe_up_many_rows(xdtype, shape):
     T, K, N, E, g = shape
-    say(f"moeUp gemm {xdtype} {shape}")
+    say(f"moeUp many rows {xdtype} {shape}")
     _check_up(T, K, N, E, g, 8, k=2, xdtype=xdtype)
 
 
 @pytest.mark.parametrize("shape", GEMM_SHAPES + GEMM_DOWN_SHAPES)
-def test_moe_down_grouped_gemm(shape):
+def test_moe_down_many_rows(shape):
     T, K, N, E, g = shape
-    say(f"moeDown gemm {shape}")
+    say(f"moeDown many rows {shape}")
     _check_down(T, K, N, E, g, 8, k=2)
+
+
+# The grouped GEMM: ragged last M-tiles, an N-tile with only part of its units
+# (N = 1032; I = 1408's half tile), one pass over the CUs and several, the
+# shortest K its ring takes (18 steps of 32 for f16 x, 12 for f32).
+UP_ON_GEMM = [(2400, 576, 1032, 8, "f16"), (2400, 576, 1032, 8, "f32"), (2400, 384, 1032, 8, "f32"),
+              (6000, 384, 1408, 4, "f32"), (6000, 576, 1408, 4, "f16")]
+# Down: whole K (the shortest, N-tiles with part of their units) and K in two
+# partial products, which the combine adds; how many is the launch's rule.
+DOWN_ON_GEMM = [(4100, 384, 1032, 8), (1024, 768, 2048, 8), (1100, 1408, 2040, 8)]
+
+
+@pytest.mark.parametrize("T,K,N,E,xdtype", UP_ON_GEMM)
+def test_moe_up_grouped_gemm(T, K, N, E, xdtype):
+    say(f"moeUp gemm {xdtype} {T} {K} {N} {E}")
+    assert expert_tiles("up", T, K, N, E, 2, xdtype)[0] == 128
+    _check_up(T, K, N, E, K, 8, k=2, xdtype=xdtype, sample=64)
+
+
+@pytest.mark.parametrize("T,K,N,E", DOWN_ON_GEMM)
+def test_moe_down_grouped_gemm(T, K, N, E):
+    say(f"moeDown gemm {T} {K} {N} {E}")
+    assert expert_tiles("down", T, N, K, E, 2, "f32")[1] == 128
+    _check_down(T, K, N, E, K, 8, k=2, sample=64)
 
 
 def _skewed_route(T, k=2):
@@ -258,16 +290,20 @@ def _skewed_route(T, k=2):
 
 
 @pytest.mark.parametrize("xdtype", ["f32", "f16"])
-def test_moe_up_gemm_empty_experts(xdtype):
-    say(f"moeUp gemm empty experts {xdtype}")
-    T = 1024
-    _check_up(T, 640, 264, 8, 640, 8, k=2, xdtype=xdtype, route=_skewed_route(T))
+@pytest.mark.parametrize("T,K,N,rows", [(1024, 640, 264, 16), (2400, 640, 1032, 128)])
+def test_moe_up_empty_experts(xdtype, T, K, N, rows):
+    say(f"moeUp empty experts {xdtype} {T} {K} {N}")
+    assert expert_tiles("up", T, K, N, 8, 2, xdtype)[0] == rows
+    _check_up(T, K, N, 8, K, 8, k=2, xdtype=xdtype, route=_skewed_route(T),
+              sample=64 if rows == 128 else None)
 
 
-def test_moe_down_gemm_empty_experts():
-    say("moeDown gemm empty experts")
-    T = 1024
-    _check_down(T, 384, 520, 8, 384, 8, k=2, route=_skewed_route(T))
+@pytest.mark.parametrize("T,K,N,rows", [(1024, 384, 520, 16), (4100, 384, 1032, 128),
+                                        (1024, 768, 2048, 128)])
+def test_moe_down_empty_experts(T, K, N, rows):
+    say(f"moeDown empty experts {T} {K} {N}")
+    assert expert_tiles("down", T, N, K, 8, 2, "f32")[1] == rows
+    _check_down(T, K, N, 8, K, 8, k=2, route=_skewed_route(T), sample=64 if rows == 128 else None)
 
 
 def test_moe_up_past_65535_rows():
@@ -436,11 +472,15 @@ def test_single_token_route_is_the_routers(d, E, k, x_dtype, calls):
 
 
 @pytest.mark.parametrize("T,E,k,x_dtype", [(64, 64, 16, "f32"), (17, 32, 8, "f16"),
-                                           (64, 128, 4, "f32"), (65, 16, 4, "f32")])
+                                           (64, 128, 4, "f32"), (65, 16, 4, "f32"),
+                                           (47, 32, 1, "f32"), (48, 64, 1, "f16"), (49, 32, 1, "f32"),
+                                           (17, 16, 1, "f16"), (12, 128, 4, "f32"), (3, 64, 16, "f16"),
+                                           (24, 130, 2, "f32")])
 def test_moe_layer_fused_router_dispatch_limits(T, E, k, x_dtype):
-    """Calls of up to 64 tokens (T·k ≤ 1024) route and dispatch in one
-    kernel whose wavefronts take several tokens each; 65 tokens take the
-    separate dispatch. Routes bit-exact, outputs at the layer bar."""
+    """Calls of up to 48 assignments route and dispatch in one kernel whose
+    wavefronts take several tokens each from 17 tokens on; above, the dispatch
+    is a kernel of its own, and from 65 tokens on so are the router's tiles.
+    Routes bit-exact, outputs at the layer bar."""
     from runntime_amd.synth import MoeConfig
     cfg = MoeConfig(f"fused_T{T}_E{E}_k{k}", T, 256, E, k, 256, x_dtype)
     say(f"moe_layer {cfg.name}")
