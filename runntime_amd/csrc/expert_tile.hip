@@ -532,9 +532,10 @@ bool expert_tile_eligible(const ExpertArgs &ea) {
 //     1000 wavefronts on it is this one (640 × 640 32 tokens 60 → 54;
 //     2048 × 1408 f16 64 tokens 232 → 121, 300 tokens 611 → 174).
 //   Row tile: as the rows an expert has on average, with room for their
-//     spread (2048 × 1408, 12 rows each: 150 with 16-row tiles, 127 with 32;
-//     24: 206, 153, 150 with 64; 48: 331, 243, 180), halved while the launch
-//     has under two blocks a CU (512 × 1024, E 8, 48 rows each: 46, 50, 60).
+//     spread (2048 × 1408, E 64, f16 x, 10 rows each: 121 with 16-row tiles, 116
+//     with 32; 12: 124, 117; 24: 201, 143, 158 with 64; 48: 316, 234, 186),
+//     halved while the launch has under two blocks a CU (512 × 1024, E 8, 48
+//     rows each: 37, 41, 57).
 int expert_tile_rows(const ExpertArgs &ea) {
   if (!expert_tile_eligible(ea) || expert_uses_gemm(ea)) return 0;
   const int max_active = ea.E < ea.A ? ea.E : ea.A;
