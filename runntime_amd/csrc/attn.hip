@@ -360,6 +360,126 @@ __device__ __forceinline__ floatx4 rope4(float4 x, float4 c, float4 s) {
                  x.w * c.w + x.z * s.w};
 }
 
+// What a wavefront of k_sdpa_mfma leaves for its keys.
+template <int NB> struct SdpaSums {
+  float mx, sum;
+  floatx4 acc[NB][4];
+};
+
+// The V operand of P·V is shared by the tile's rows, and 0 times an infinity
+// or a NaN of a key that a row does not see is NaN. Such a NaN stays in the sums,
+// so k_sdpa_mfma's loop needs no test: a wavefront that ends with one walks its
+// keys again here, P·V for one row after the other with the V it does not see
+// zeroed. Nothing is kept for it: it reads the kernel's arguments again and loads
+// where it multiplies, so that the loop keeps its registers and its schedule.
+// (Written with the loop's own parts it cost every call 3 to 10%, 77 rows 9.0 →
+// 9.8 µs; so 64 rows 6.6, 6.6; 300 rows 18.3, 18.4; 4096 rows 105, 105.)
+template <typename T, int NB, int NT, bool ROPE>
+__device__ __forceinline__ SdpaSums<NB> sdpa_by_rows(int h, int lo, int hi, int blo, int bhi,
+                                                     int c_first, int c_last) {
+  constexpr int HD = 64 * NB, NS = HD / 16, KC = 16 * NT;
+  // AttnArgs is k_sdpa_mfma's first argument.
+  typedef const __attribute__((address_space(4))) AttnArgs *KernArgs;
+  uint64_t kp0 = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+  int lane = threadIdx.x & (WAVE - 1);
+  asm("" : "+s"(kp0), "+v"(lane));
+  const KernArgs a = (KernArgs)kp0;
+  const int row0 = blockIdx.x * 16, kvh = h / (a->q_heads / a->kv_heads);
+  const int m = lane & 15, g = lane >> 4;
+  const int row = min(row0 + m, a->q_len - 1);
+  const T *qp = (const T *)a->q + (int64_t)row * a->q_rs + (int64_t)h * HD;
+  const T *kp = (const T *)a->k + (int64_t)kvh * HD;
+  const T *vp = (const T *)a->v + (int64_t)kvh * HD;
+  auto roped = [&](const T *p, int64_t r, int x) {
+    const float4 v = Ld4<T>::at(p + x);
+    if constexpr (ROPE)
+      return rope4(v, *(const float4 *)(a->rope_cos + r * HD + x),
+                   *(const float4 *)(a->rope_sin + r * HD + x));
+    else
+      return floatx4{v.x, v.y, v.z, v.w};
+  };
+  SdpaSums<NB> o;
+  o.mx = -INFINITY;
+  o.sum = 0.f;
+#pragma unroll
+  for (int b = 0; b < NB; b++)
+#pragma unroll
+    for (int c = 0; c < 4; c++) o.acc[b][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int st = c_first; st < c_last; st++) {
+    const int k0 = blo + st * KC;
+    floatx4 sc[NT];
+#pragma unroll
+    for (int n = 0; n < NT; n++) {
+      const int64_t key = min(k0 + 16 * n + m, bhi);
+      sc[n] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+      for (int s = 0; s < NS; s++) {
+        const int x = 16 * s + 4 * g;
+        const floatx4 k4 = roped(kp + key * a->k_rs, key, x), q4 = roped(qp, row, x);
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          sc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[j], q4[j], sc[n], 0, 0, 0);
+      }
+    }
+    auto key_of = [&](int n, int j) { return k0 + 16 * n + 4 * g + j; };
+    float top = -INFINITY;
+#pragma unroll
+    for (int n = 0; n < NT; n++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int key = key_of(n, j);
+        if (a->has_kb && key >= a->kb_start && key < a->kb_end) sc[n][j] += a->kb_value;
+        sc[n][j] = key >= lo && key <= hi ? sc[n][j] : -INFINITY;
+        top = fmaxf(top, sc[n][j]);
+      }
+    top = fmaxf(top, __shfl_xor(top, 16));
+    top = fmaxf(top, __shfl_xor(top, 32));
+    const float mn = fmaxf(o.mx, top);
+    const float base = mn == -INFINITY ? 0.f : mn;
+    const float scale = o.mx == -INFINITY ? 0.f : expf(o.mx - base);
+    float add = 0.f;
+#pragma unroll
+    for (int n = 0; n < NT; n++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int key = key_of(n, j);
+        sc[n][j] = key >= lo && key <= hi ? expf(sc[n][j] - base) : 0.f;
+        add += sc[n][j];
+      }
+    add += __shfl_xor(add, 16);
+    add += __shfl_xor(add, 32);
+    o.sum = o.sum * scale + add;
+    o.mx = mn;
+#pragma unroll 1
+    for (int r = 0; r < 16; r++) {
+      const int rlo = __builtin_amdgcn_readlane(lo, r), rhi = __builtin_amdgcn_readlane(hi, r);
+#pragma unroll
+      for (int b = 0; b < NB; b++) {
+        floatx4 pv[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) pv[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int n = 0; n < NT; n++)
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            const int key = key_of(n, j);
+            const float4 v = Ld4<T>::at(vp + (int64_t)min(key, bhi) * a->v_rs + 64 * b + 4 * m);
+            const bool in = key >= rlo && key <= rhi;
+            pv[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? v.x : 0.f, sc[n][j], pv[0], 0, 0, 0);
+            pv[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? v.y : 0.f, sc[n][j], pv[1], 0, 0, 0);
+            pv[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? v.z : 0.f, sc[n][j], pv[2], 0, 0, 0);
+            pv[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? v.w : 0.f, sc[n][j], pv[3], 0, 0, 0);
+          }
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+          if (m == r) o.acc[b][c] = o.acc[b][c] * scale + pv[c];
+      }
+    }
+  }
+  return o;
+}
+
 template <typename T, int NB, int NT, bool ROPE>  // head_dim 64·NB, 16·NT keys a step
 __global__ __launch_bounds__(512) void k_sdpa_mfma(AttnArgs a, int hw, int ksplit) {
   constexpr int HD = 64 * NB, NS = HD / 16;
@@ -456,98 +576,81 @@ __global__ __launch_bounds__(512) void k_sdpa_mfma(AttnArgs a, int hw, int kspli
   for (int b = 0; b < NB; b++)
 #pragma unroll
     for (int c = 0; c < 4; c++) acc[b][c] = floatx4{0.f, 0.f, 0.f, 0.f};
-  auto scores = [&](const KTile &kt, floatx4 (&sc)[NT]) {
-#pragma unroll
-    for (int n = 0; n < NT; n++) {
-      // two chains: halves the dependent MFMA latency
-      floatx4 s0 = floatx4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
-#pragma unroll
-      for (int s = 0; s < NS; s++) {
-        floatx4 k4;
-        if constexpr (ROPE)
-          k4 = rope4(kt.k[n][s], kt.c[n][s], kt.s[n][s]);
-        else
-          k4 = floatx4{kt.k[n][s].x, kt.k[n][s].y, kt.k[n][s].z, kt.k[n][s].w};
-        s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[0], q[s][0], s0, 0, 0, 0);
-        s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[1], q[s][1], s1, 0, 0, 0);
-        s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[2], q[s][2], s0, 0, 0, 0);
-        s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[3], q[s][3], s1, 0, 0, 0);
-      }
-      sc[n] = s0 + s1;
-    }
-  };
-  // Scores of step st to probabilities under the running max; returns the
-  // factor for what was summed before.
-  auto softmax = [&](int st, floatx4 (&sc)[NT]) -> float {
-    const int key0 = blo + st * KC + 4 * g;
-    float top = -INFINITY;
-#pragma unroll
-    for (int n = 0; n < NT; n++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const int key = key0 + 16 * n + j;
-        float x = sc[n][j];
-        if (a.has_kb && key >= a.kb_start && key < a.kb_end) x += a.kb_value;
-        x = key >= lo && key <= hi ? x : -INFINITY;
-        sc[n][j] = x;
-        top = fmaxf(top, x);
-      }
-    top = fmaxf(top, __shfl_xor(top, 16));
-    top = fmaxf(top, __shfl_xor(top, 32));
-    const float mn = fmaxf(mx, top);
-    const float base = mn == -INFINITY ? 0.f : mn;  // nothing seen yet
-    const float scale = mx == -INFINITY ? 0.f : expf(mx - base);
-    float add = 0.f;
-#pragma unroll
-    for (int n = 0; n < NT; n++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const int key = key0 + 16 * n + j;
-        const float p = key >= lo && key <= hi ? expf(sc[n][j] - base) : 0.f;
-        sc[n][j] = p;
-        add += p;
-      }
-    add += __shfl_xor(add, 16);
-    add += __shfl_xor(add, 32);
-    sum = sum * scale + add;
-    mx = mn;
-    return scale;
-  };
-  // P·V of head columns (b, c); keys outside klo .. khi count as V = 0.
-  auto pv = [&](int b, int c, const floatx4 (&sc)[NT], bool masked, int key0, int klo, int khi) {
-    floatx4 o = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int n = 0; n < NT; n++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const float4 &vv = v[n][j][b];
-        float ve = c == 0 ? vv.x : c == 1 ? vv.y : c == 2 ? vv.z : vv.w;
-        if (masked) ve = key0 + 16 * n + j >= klo && key0 + 16 * n + j <= khi ? ve : 0.f;
-        o = __builtin_amdgcn_mfma_f32_16x16x4f32(ve, sc[n][j], o, 0, 0, 0);
-      }
-    return o;
-  };
   if (c_first < c_last) {  // then blo ≤ bhi: every address is a key's
     KTile kt;
     load_k(c_first, kt);
     load_v(c_first);
     for (int st = c_first; st < c_last; st++) {
       floatx4 sc[NT];
-      scores(kt, sc);
+#pragma unroll
+      for (int n = 0; n < NT; n++) {
+        // two chains: halves the dependent MFMA latency
+        floatx4 s0 = floatx4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+          floatx4 k4;
+          if constexpr (ROPE)
+            k4 = rope4(kt.k[n][s], kt.c[n][s], kt.s[n][s]);
+          else
+            k4 = floatx4{kt.k[n][s].x, kt.k[n][s].y, kt.k[n][s].z, kt.k[n][s].w};
+          s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[0], q[s][0], s0, 0, 0, 0);
+          s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[1], q[s][1], s1, 0, 0, 0);
+          s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[2], q[s][2], s0, 0, 0, 0);
+          s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[3], q[s][3], s1, 0, 0, 0);
+        }
+        sc[n] = s0 + s1;
+      }
       load_k(min(st + 1, c_last - 1), kt);  // lands under the softmax and P·V
-      const float scale = softmax(st, sc);
+      const int key0 = blo + st * KC + 4 * g;
+      float top = -INFINITY;
+#pragma unroll
+      for (int n = 0; n < NT; n++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const int key = key0 + 16 * n + j;
+          float x = sc[n][j];
+          if (a.has_kb && key >= a.kb_start && key < a.kb_end) x += a.kb_value;
+          x = key >= lo && key <= hi ? x : -INFINITY;
+          sc[n][j] = x;
+          top = fmaxf(top, x);
+        }
+      top = fmaxf(top, __shfl_xor(top, 16));
+      top = fmaxf(top, __shfl_xor(top, 32));
+      const float mn = fmaxf(mx, top);
+      const float base = mn == -INFINITY ? 0.f : mn;  // nothing seen yet
+      const float scale = mx == -INFINITY ? 0.f : expf(mx - base);
+      float add = 0.f;
+#pragma unroll
+      for (int n = 0; n < NT; n++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const int key = key0 + 16 * n + j;
+          const float p = key >= lo && key <= hi ? expf(sc[n][j] - base) : 0.f;
+          sc[n][j] = p;
+          add += p;
+        }
+      add += __shfl_xor(add, 16);
+      add += __shfl_xor(add, 32);
+      sum = sum * scale + add;
+      mx = mn;
 #pragma unroll
       for (int b = 0; b < NB; b++)
 #pragma unroll
-        for (int c = 0; c < 4; c++)
-          acc[b][c] = acc[b][c] * scale + pv(b, c, sc, false, 0, 0, 0);
+        for (int c = 0; c < 4; c++) {
+          floatx4 o = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int n = 0; n < NT; n++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+              const float4 &vv = v[n][j][b];
+              const float ve = c == 0 ? vv.x : c == 1 ? vv.y : c == 2 ? vv.z : vv.w;
+              o = __builtin_amdgcn_mfma_f32_16x16x4f32(ve, sc[n][j], o, 0, 0, 0);
+            }
+          acc[b][c] = acc[b][c] * scale + o;
+        }
       load_v(min(st + 1, c_last - 1));
     }
   }
-  // The V operand is shared by the tile's rows, and 0 times an infinity or a
-  // NaN of a key that a row does not see is NaN. Such a NaN stays in acc, so
-  // the loop above needs no test; where one came out, the keys are walked
-  // again, P·V for one row after the other with the V it does not see zeroed.
   bool nan = false;
 #pragma unroll
   for (int b = 0; b < NB; b++)
@@ -555,35 +658,15 @@ __global__ __launch_bounds__(512) void k_sdpa_mfma(AttnArgs a, int hw, int kspli
     for (int c = 0; c < 4; c++)
 #pragma unroll
       for (int i = 0; i < 4; i++) nan |= acc[b][c][i] != acc[b][c][i];
-  if (__any(nan)) {
-    mx = -INFINITY;
-    sum = 0.f;
+  if (__builtin_expect(__any(nan), 0)) {
+    const SdpaSums<NB> o =
+        sdpa_by_rows<T, NB, NT, ROPE>(h, lo, hi, blo, bhi, c_first, c_last);
+    mx = o.mx;
+    sum = o.sum;
 #pragma unroll
     for (int b = 0; b < NB; b++)
 #pragma unroll
-      for (int c = 0; c < 4; c++) acc[b][c] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int st = c_first; st < c_last; st++) {
-      floatx4 sc[NT];
-      {
-        KTile kt;
-        load_k(st, kt);
-        scores(kt, sc);
-      }
-      const float scale = softmax(st, sc);
-      load_v(st);
-#pragma unroll 1
-      for (int r = 0; r < 16; r++) {
-        const int rlo = __builtin_amdgcn_readlane(lo, r), rhi = __builtin_amdgcn_readlane(hi, r);
-#pragma unroll
-        for (int b = 0; b < NB; b++)
-#pragma unroll
-          for (int c = 0; c < 4; c++) {
-            const floatx4 o = pv(b, c, sc, true, blo + st * KC + 4 * g, rlo, rhi);
-            if (m == r) acc[b][c] = acc[b][c] * scale + o;
-          }
-      }
-    }
+      for (int c = 0; c < 4; c++) acc[b][c] = o.acc[b][c];
   }
   // acc[b][c][i]: row `row`, head column 64b + 16g + 4i + c.
   if (ksplit > 1) {
