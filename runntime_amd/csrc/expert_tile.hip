@@ -31,7 +31,7 @@
 //
 // Bound by the weight stream while an expert has up to ~32 rows, by the
 // int8 → f16 conversions and MFMAs above. Measured (2048 × 1408, E 64, 300
-// tokens, top-8, f16 x): layer 611 → 174 µs against the skinny kernel (up 397,
+// tokens, top-8, f16 x): layer 611 → 168 µs against the skinny kernel (up 397,
 // down 208), which takes 16 rows at a time and streams (and converts) the
 // weights once for each.
 // Ring of 4 load steps: 8 is no faster with plain scales and spills with
@@ -530,7 +530,7 @@ bool expert_tile_eligible(const ExpertArgs &ea) {
 //     the skinny kernel, which splits K over wavefronts (one token: 33 there,
 //     36 here; 2048 × 1408 two tokens 57, 60), from three rows an expert or
 //     1000 wavefronts on it is this one (640 × 640 32 tokens 60 → 54;
-//     2048 × 1408 f16 64 tokens 232 → 121, 300 tokens 611 → 174).
+//     2048 × 1408 f16 64 tokens 232 → 121, 300 tokens 611 → 168).
 //   Row tile: as the rows an expert has on average, with room for their
 //     spread (2048 × 1408, E 64, f16 x, 10 rows each: 121 with 16-row tiles, 116
 //     with 32; 12: 124, 117; 24: 201, 143, 158 with 64; 48: 316, 234, 186),
