@@ -766,7 +766,7 @@ int launch_sdpa(AttnArgs a, hipStream_t s) {
     // Keys of a row tile: the window and 15 more rows, at most kv_len.
     const int64_t span = a.window_left < 0 || a.window_right < 0
                              ? a.kv_len
-                             : std::min((int64_t)a.kv_len, (int64_t)(a.window_left + a.window_right + 16));
+                             : std::min<int64_t>(a.kv_len, a.window_left + a.window_right + 16);
     const int kc = a.head_dim == 64 ? 32 : 16;
     const int64_t nstep = (span + kc - 1) / kc;
     const int64_t tiles = ((int64_t)a.q_len + 15) / 16;

@@ -1021,6 +1021,10 @@ extern "C" int moe_linear(moe_ctx *ctx, const float *x, const float *w, const fl
   return after_launch("linear");
 }
 
+// Negative: unbounded. So is a window that reaches past every 32-bit position,
+// and the kernels' sums of positions and windows stay in 64 bits.
+static int64_t lower_window(int64_t w) { return w < 0 || w > UINT32_MAX ? -1 : w; }
+
 extern "C" int moe_attention(moe_ctx *ctx, const void *qkv, moe_dtype dtype, int T, int q_heads,
                              int kv_heads, int head_dim, int64_t window_left,
                              int64_t window_right, const float *sinks, const float *cos_t,
@@ -1048,8 +1052,8 @@ extern "C" int moe_attention(moe_ctx *ctx, const void *qkv, moe_dtype dtype, int
   a.q_heads = q_heads;
   a.kv_heads = kv_heads;
   a.head_dim = head_dim;
-  a.window_left = window_left < 0 ? -1 : window_left;
-  a.window_right = window_right < 0 ? -1 : window_right;
+  a.window_left = lower_window(window_left);
+  a.window_right = lower_window(window_right);
   a.sinks = sinks;
   a.rope_cos = cos_t;
   a.rope_sin = sin_t;
@@ -1122,8 +1126,8 @@ extern "C" int moe_sdpa(moe_ctx *ctx, moe_dtype dtype, const void *q, int64_t q_
   a.q_heads = q_heads;
   a.kv_heads = kv_heads;
   a.head_dim = head_dim;
-  a.window_left = window_left < 0 ? -1 : window_left;
-  a.window_right = window_right < 0 ? -1 : window_right;
+  a.window_left = lower_window(window_left);
+  a.window_right = lower_window(window_right);
   a.q_pos_offset = q_pos_offset;
   a.sinks = sinks;
   a.segs = segments;

@@ -208,6 +208,28 @@ def test_sdpa_keeps_infinities_from_rows_that_do_not_see_them(dtype, n, qh, kh, 
                                rtol=1e-4 if dtype == "f32" else 1e-3)
 
 
+@pytest.mark.parametrize("hd", [64, 32])  # k_sdpa_mfma, k_sdpa
+def test_sdpa_windows_of_any_size(hd):
+    """The C entry takes 64-bit windows: one past every key is unbounded, up to
+    the largest, where a position plus the window would pass 64 bits."""
+    print(f"sdpa windows {hd}", flush=True)
+    from runntime_amd.core import _sdpa_launch
+    n = 40
+    g = torch.Generator(device=DEV).manual_seed(hd)
+    q, k, v = (torch.randn((n, hd), generator=g, device=DEV) for _ in range(3))
+
+    def run(left, right):
+        return _sdpa_launch(q.device, q.data_ptr(), hd, k.data_ptr(), hd, v.data_ptr(), hd, n, n, 1, 1,
+                            hd, left, right, 0, None, None, None, torch.float32)
+    every, behind = run(-1, -1), run(-1, 2)
+    want = torch.softmax(q.double() @ k.double().T, -1) @ v.double()
+    torch.testing.assert_close(every.double(), want, atol=2e-5, rtol=1e-4)
+    for big in (n, (1 << 31) - 1, 1 << 31, (1 << 32) - 1, 1 << 32, (1 << 63) - 1):
+        # a bounded side may split the keys over wavefronts otherwise
+        torch.testing.assert_close(run(big, big), every, atol=4e-5, rtol=1e-4)
+        torch.testing.assert_close(run(big, 2), behind, atol=4e-5, rtol=1e-4)
+
+
 # Rows per expert from one to a second 32-row tile; K whole steps, past one by
 # 4, and odd; N a partial column block; few blocks, and 16-row tiles of 512 and
 # more (no step ahead).
