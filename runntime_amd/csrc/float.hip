@@ -150,8 +150,14 @@ __global__ __launch_bounds__(FWAVES *WAVE) __attribute__((amdgpu_waves_per_eu(4)
     wv4 b[4];
   };
   // Addresses of a stay inside its rows: a step past the last reads that one
-  // (not used), a k past K reads k = 0.
+  // (not used), a k past K reads k = 0. Of W, a step past the wavefront's share
+  // reads nothing: with five steps a share, two of seven were read for no use
+  // (block of 8 tokens, f32 54.5 → 51.0 µs, f16 44.3 → 43.6; 68.5 and 51.6 with
+  // the VALU gathers; the same tokens again and again, weights in cache, 53.9 →
+  // 50.3 and 44.5 → 43.9, 48.7 and 42.0 with the gathers). Two steps ahead: 52.2
+  // and 45.1, three 54.0 and 47.6.
   auto load = [&](int s, Step &d) {
+    const bool past = s >= s1;
     s = min(s, steps - 1);
     const int k = s * FSTEP + 4 * kq;
     if constexpr (KF == K_WIDE) {
@@ -163,7 +169,7 @@ __global__ __launch_bounds__(FWAVES *WAVE) __attribute__((amdgpu_waves_per_eu(4)
         for (int c = 0; c < 4; c++) d.b[j][c] = ok ? v[c] : (WT)0;
       }
     } else {
-      const int left = KF == K_STEPS ? FSTEP : min(FSTEP, p.K - s * FSTEP);
+      const int left = past ? 0 : KF == K_STEPS ? FSTEP : min(FSTEP, p.K - s * FSTEP);
       const __amdgpu_buffer_rsrc_t wr =
           rows_rsrc(w + (int64_t)s * FSTEP * p.N, left * p.N * (int)sizeof(WT));
 #pragma unroll
