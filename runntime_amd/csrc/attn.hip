@@ -330,8 +330,8 @@ __global__ __launch_bounds__(AW *WAVE) void k_sdpa(AttnArgs a) {
 // in order (short sequences, few heads).
 // Bound by latency and L1 (each wavefront reads K, V and the rope tables of
 // its keys, 32 KB a step). Against k_sdpa below (f32 VALU, K and V through
-// LDS), 14 heads over 2 kv heads of 64, rope, window ±128: 64 rows 11.4 → 7.5
-// µs, 1500 rows 126 → 51 (27 TFLOP/s), 4096 rows 280 → 78.
+// LDS), 14 heads over 2 kv heads of 64, rope, window ±128: 64 rows 9.8 → 7.4
+// µs, 1500 rows 123 → 50 (27 TFLOP/s), 4096 rows 308 → 108.
 template <typename T> struct Ld4;
 template <> struct Ld4<float> {
   static __device__ __forceinline__ float4 at(const float *p) { return *(const float4 *)p; }

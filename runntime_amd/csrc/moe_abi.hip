@@ -723,8 +723,8 @@ static int layer_impl(const char *op, moe_ctx *ctx, int calls, const moe_call_st
     }
   } else {
     dn.parts = 1;
-    // Both on the decode kernels: act in dispatch order too (f32), so down
-    // stages its rows without waiting on the permutation.
+    // Neither on the grouped GEMM (decode kernels, row tiles): act in dispatch
+    // order too (f32), so down stages its rows without gathering them.
     if (!expert_uses_gemm(up) && !expert_uses_gemm(dn)) up.dispatch_order = dn.dispatch_order = 1;
   }
   dn.out_cs = (int64_t)dn.parts * A * d;
@@ -735,8 +735,8 @@ static int layer_impl(const char *op, moe_ctx *ctx, int calls, const moe_call_st
   // staging for calls of at most FUSED_T tokens (the router's chunk kernel
   // computes and leaves each token's inverse RMS in the xn slot); for larger
   // calls (the register-tiled router, whose many blocks per token tile would
-  // each recompute it) and for the grouped GEMM (loads straight into LDS), a
-  // normalised copy xn.
+  // each recompute it), for the row tiles and for the grouped GEMM (loads
+  // straight into LDS), a normalised copy xn.
   const bool stage_norm = norm && T <= FUSED_T && expert_stages_norm(up);
   if ((rc = plan_ws(ctx, calls, T, k, E, route_out ? 0 : (size_t)T * 2 * k,
                     router_partial_floats(T, d, E), act_floats, (size_t)dn.parts * A * d, L,
